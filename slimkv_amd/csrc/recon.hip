@@ -24,6 +24,9 @@ struct ReconParams {
     const float* cos; const float* sin; int64_t rope_rows;
     const int64_t* positions; int64_t pos_sb;                 // [B, n] or null
     int B, n, R, Hkv, blockdiag, k_lo_step;                   // k_lo_step: per-head latent slice width
+    int in16, out16;                                          // latent and W / output rows 16-byte aligned
+    int tables16;                                             // RoPE tables 16-byte aligned
+    int row_frags;                                            // 16-row groups a tile of the wide kernel
 };
 
 constexpr int kReconWaves = 4;
@@ -102,7 +105,8 @@ recon_kernel(ReconParams p) {
 // Streaming variant for narrow contractions (kw <= 64): the wavefront keeps its
 // head's W tile (A operand, 128 x kw) in registers and walks 16-row tiles with
 // the next tile's latent rows already in flight, so W is read once per
-// wavefront instead of once per tile.  Same epilogue as recon_kernel.
+// wavefront instead of once per tile.  Same epilogue as recon_kernel, which
+// stays for these widths with RoPE tables off a 16-byte boundary.
 template <int KSTEPS>
 __device__ __forceinline__ void recon_stream_body(const ReconParams& p, int segs, int block) {
     constexpr int D = 128;
@@ -208,9 +212,244 @@ recon_stream_pair_kernel(ReconParams p0, ReconParams p1, int segs0, int segs1, i
     else recon_stream_body<KSTEPS>(p1, segs1, blockIdx.x - blocks0);
 }
 
+// Wide contractions (kw >= 128: up-projections that couple every KV head).  A
+// workgroup owns a head's 128 features and walks tiles of 16 RT rows; wave w
+// holds the W rows of its own 32 features over the whole contraction in
+// registers (64 VGPRs at kw 256) and multiplies them with the tile's latent
+// rows on the 16x16x32 MFMA.  W (once a workgroup) and the latent rows go
+// through LDS: an operand read straight from memory touches sixteen rows per
+// sixteen lanes, and the cache's line lookups bound the kernel (7936 rows of
+// width 256 on 8 heads: 26.9 us that way against 12.4 with whole rows read in
+// lane order, 69.5 with W also read again for every tile; two problems of 256
+// rows: 39 us as two such launches, 5.0 as one of these; the write of the
+// rebuilt rows alone takes 3).  16-byte chunk c of row r sits at chunk
+// c ^ (r & 7) of its LDS row, so eight lanes that read one chunk of eight
+// rows meet eight different bank groups.
+//
+// Without RoPE the wave's features are 32w + 8*grp + [0, 8) a lane: the two A
+// operands interleave the rows in fours, so a lane stores 16 contiguous
+// bytes.  With RoPE they are 16w and 64 + 16w + [0, 16), so d and d + 64 share
+// a lane for the rotation.
+// AL16: latent and W rows 16-byte aligned, else 8-byte loads.
+template <bool AL16>
+__device__ __forceinline__ u32x4 load_piece(const uint16_t* src) {
+    if constexpr (AL16) {
+        return *reinterpret_cast<const u32x4*>(src);
+    } else {
+        const u32x2 lo = *reinterpret_cast<const u32x2*>(src);
+        const u32x2 hi = *reinterpret_cast<const u32x2*>(src + 4);
+        return u32x4{lo.x, lo.y, hi.x, hi.y};
+    }
+}
+
+// LDS of a workgroup: two tiles of 32 rows, or 16 W rows for each wave.
+template <int KS>
+struct WideLds {
+    static constexpr int bytes = 2 * 32 * KS * 64;
+};
+
+template <int KS, int RT, bool ROPE, bool AL16>
+__device__ __forceinline__ void recon_wide_body(const ReconParams& p, int segs, int block, char* lds) {
+    constexpr int D = 128;
+    constexpr int C = 4 * KS;                 // 16-byte chunks of a row
+    constexpr int ROWS = 16 * RT;
+    constexpr int CHUNKS = ROWS * C;
+    constexpr int PIECES = (CHUNKS + 255) / 256;   // chunks a thread stages of a tile
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int col = lane & 15, grp = lane >> 4;
+    // Row segments fastest over the 8 XCDs (workgroups are dealt to them in
+    // turn), heads next: an XCD's L2 then holds the rows of its segments for
+    // every head.
+    int h, seg;
+    const int b = block / (p.Hkv * segs);
+    const int rest = block % (p.Hkv * segs);
+    if (segs % 8 == 0) {
+        h = (rest / 8) % p.Hkv;
+        seg = rest / (8 * p.Hkv) * 8 + rest % 8;
+    } else {
+        h = rest % p.Hkv;
+        seg = rest / p.Hkv;
+    }
+    const int tiles = (p.n + ROWS - 1) / ROWS;
+    const int k_lo = p.blockdiag ? h * p.k_lo_step : 0;
+    auto feature = [&](int f, int r) { return ROPE ? 64 * f + 16 * wave + r : 32 * wave + 8 * (r >> 2) + 4 * f + (r & 3); };
+    auto slot = [](int row, int chunk) { return (row * C + (chunk ^ (row & 7))) * 16; };
+
+    int tile = seg;
+    if (tile >= tiles) return;                // the whole workgroup
+    const uint16_t* lbase = p.latent + (int64_t)b * p.l_sb + k_lo;
+    u32x4 stage[PIECES];
+    auto fetch = [&](int t) {
+#pragma unroll
+        for (int i = 0; i < PIECES; ++i) {
+            const int id = min(256 * i + (int)threadIdx.x, CHUNKS - 1);
+            stage[i] = load_piece<AL16>(lbase + (int64_t)min(t * ROWS + id / C, p.n - 1) * p.l_sn + 8 * (id % C));
+        }
+    };
+    auto put = [&](char* buf) {
+#pragma unroll
+        for (int i = 0; i < PIECES; ++i) {
+            const int id = 256 * i + threadIdx.x;
+            if (CHUNKS % 256 == 0 || id < CHUNKS) *reinterpret_cast<u32x4*>(buf + slot(id / C, id % C)) = stage[i];
+        }
+    };
+    auto operand = [&](const char* buf, int row, int ks) {
+        return *reinterpret_cast<const u32x4*>(buf + slot(row, 4 * ks + grp));
+    };
+
+    // W: every load of both operands and of the first tile goes out at once;
+    // then each wave stages the 16 rows of one operand at a time in its own
+    // part of the LDS.
+    u32x4 wa[2][KS];
+    char* own = lds + wave * 16 * C * 16;
+    {
+        u32x4 w[2][C / 4];
+#pragma unroll
+        for (int f = 0; f < 2; ++f)
+#pragma unroll
+            for (int i = 0; i < C / 4; ++i) {
+                const int id = 64 * i + lane;
+                w[f][i] = load_piece<AL16>(p.w + ((int64_t)h * D + feature(f, id / C)) * p.w_ld + k_lo + 8 * (id % C));
+            }
+        fetch(tile);
+#pragma unroll
+        for (int f = 0; f < 2; ++f) {
+#pragma unroll
+            for (int i = 0; i < C / 4; ++i) {
+                const int id = 64 * i + lane;
+                *reinterpret_cast<u32x4*>(own + slot(id / C, id % C)) = w[f][i];
+            }
+            __syncthreads();
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) wa[f][ks] = operand(own, col, ks);
+            __syncthreads();
+        }
+    }
+    float bias[2][4];
+#pragma unroll
+    for (int f = 0; f < 2; ++f)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) bias[f][i] = p.bias ? bf16_to_f32(p.bias[(int64_t)h * D + feature(f, 4 * grp + i)]) : 0.f;
+
+    // The RoPE table pieces of a lane's row, loaded before the tile's products.
+    struct RopePiece {
+        float4 c[2], s[2];
+    };
+    auto load_rope = [&](RopePiece& t, int row) {
+        const int64_t pos = clamp_i64(p.positions[(int64_t)b * p.pos_sb + min(row, p.n - 1)], 0, p.rope_rows - 1);
+#pragma unroll
+        for (int f = 0; f < 2; ++f) {
+            const float* cr = p.cos + pos * D + feature(f, 4 * grp);
+            const float* sr = p.sin + pos * D + feature(f, 4 * grp);
+            if (p.tables16) {
+                t.c[f] = *reinterpret_cast<const float4*>(cr);
+                t.s[f] = *reinterpret_cast<const float4*>(sr);
+            } else {
+                t.c[f] = make_float4(cr[0], cr[1], cr[2], cr[3]);
+                t.s[f] = make_float4(sr[0], sr[1], sr[2], sr[3]);
+            }
+        }
+    };
+    auto finish = [&](const v4f (&acc)[2], const RopePiece& t, int row) {
+        if (row >= p.n) return;
+        float x[2][4];
+#pragma unroll
+        for (int f = 0; f < 2; ++f)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) x[f][i] = round_bf16_hw(p.bias ? acc[f][i] + bias[f][i] : acc[f][i]);
+        const int64_t dst = p.dst_rows ? p.dst_rows[row] : row;
+        uint16_t* orow = p.out + (int64_t)b * p.o_sb + dst * p.o_sn + (int64_t)h * p.o_sh;
+        if constexpr (ROPE) {
+#pragma unroll
+            for (int f = 0; f < 2; ++f) {
+                const float cv[4] = {t.c[f].x, t.c[f].y, t.c[f].z, t.c[f].w}, sv[4] = {t.s[f].x, t.s[f].y, t.s[f].z, t.s[f].w};
+                float y[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const float partner = f == 0 ? -x[1][i] : x[0][i];
+                    y[i] = round_bf16_hw(x[f][i] * round_bf16_hw(cv[i])) + round_bf16_hw(partner * round_bf16_hw(sv[i]));
+                }
+                *reinterpret_cast<u32x2*>(orow + feature(f, 4 * grp)) = u32x2{pack_bf16(y[0], y[1]), pack_bf16(y[2], y[3])};
+            }
+        } else {
+            const u32x4 w = {pack_bf16(x[0][0], x[0][1]), pack_bf16(x[0][2], x[0][3]), pack_bf16(x[1][0], x[1][1]),
+                             pack_bf16(x[1][2], x[1][3])};
+            uint16_t* o = orow + 32 * wave + 8 * grp;
+            if (p.out16) {
+                *reinterpret_cast<u32x4*>(o) = w;
+            } else {
+                *reinterpret_cast<u32x2*>(o) = u32x2{w.x, w.y};
+                *reinterpret_cast<u32x2*>(o + 4) = u32x2{w.z, w.w};
+            }
+        }
+    };
+    // Double-buffered tiles, one barrier a tile: a wave writes buffer `at`
+    // only after the barrier that every wave reached past its reads of it.
+    for (int at = 0; tile < tiles; tile += segs, at ^= 1) {
+        char* buf = lds + at * 32 * C * 16;
+        put(buf);
+        __syncthreads();
+        RopePiece rope[RT];
+        if constexpr (ROPE) {
+#pragma unroll
+            for (int r = 0; r < RT; ++r) load_rope(rope[r], tile * ROWS + 16 * r + col);
+        }
+        if (tile + segs < tiles) fetch(tile + segs);
+        v4f acc[RT][2];
+#pragma unroll
+        for (int r = 0; r < RT; ++r) acc[r][0] = acc[r][1] = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+            for (int r = 0; r < RT; ++r) {
+                const u32x4 lr = operand(buf, 16 * r + col, ks);
+#pragma unroll
+                for (int f = 0; f < 2; ++f) acc[r][f] = mfma32(wa[f][ks], lr, acc[r][f]);
+            }
+#pragma unroll
+        for (int r = 0; r < RT; ++r) finish(acc[r], rope[r], tile * ROWS + 16 * r + col);
+    }
+}
+
+template <int KS, int RT, bool ROPE, bool AL16>
+__global__ void __launch_bounds__(kReconWaves * 64) __attribute__((amdgpu_waves_per_eu(2)))
+recon_wide_kernel(ReconParams p, int segs) {
+    __shared__ __attribute__((aligned(16))) char lds[WideLds<KS>::bytes];
+    recon_wide_body<KS, RT, ROPE, AL16>(p, segs, blockIdx.x, lds);
+}
+
+// Two reconstructions of one width in one launch, as recon_stream_pair_kernel.
+template <int KS, int RT>
+__global__ void __launch_bounds__(kReconWaves * 64) __attribute__((amdgpu_waves_per_eu(2)))
+recon_wide_pair_kernel(ReconParams p0, ReconParams p1, int segs0, int segs1, int blocks0) {
+    __shared__ __attribute__((aligned(16))) char lds[WideLds<KS>::bytes];
+    if ((int)blockIdx.x < blocks0) recon_wide_body<KS, RT, false, true>(p0, segs0, blockIdx.x, lds);
+    else recon_wide_body<KS, RT, false, true>(p1, segs1, blockIdx.x - blocks0, lds);
+}
+
 namespace {
 bool al4(int64_t x) { return (x & 3) == 0; }
 bool pal8(const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 7) == 0; }
+bool al8(int64_t x) { return (x & 7) == 0; }
+bool pal16(const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15) == 0; }
+
+template <int KS, int RT>
+hipError_t launch_wide_rt(const ReconParams& p, int segs, hipStream_t st) {
+    const dim3 grid(p.B * p.Hkv * segs), block(kReconWaves * 64);
+    if (p.positions) {
+        if (p.in16) hipLaunchKernelGGL((recon_wide_kernel<KS, RT, true, true>), grid, block, 0, st, p, segs);
+        else hipLaunchKernelGGL((recon_wide_kernel<KS, RT, true, false>), grid, block, 0, st, p, segs);
+    } else {
+        if (p.in16) hipLaunchKernelGGL((recon_wide_kernel<KS, RT, false, true>), grid, block, 0, st, p, segs);
+        else hipLaunchKernelGGL((recon_wide_kernel<KS, RT, false, false>), grid, block, 0, st, p, segs);
+    }
+    return hipGetLastError();
+}
+
+template <int KS>
+hipError_t launch_wide(const ReconParams& p, int segs, hipStream_t st) {
+    return p.row_frags == 1 ? launch_wide_rt<KS, 1>(p, segs, st) : launch_wide_rt<KS, 2>(p, segs, st);
+}
 
 template <int K>
 hipError_t launch_recon(const ReconParams& p, int grid, hipStream_t st) {
@@ -225,9 +464,14 @@ hipError_t launch_stream(const ReconParams& p, int segs, hipStream_t st) {
 }
 }  // namespace
 
+// Workgroups of a wide reconstruction: each loads its head's W once, so few of
+// them, but the CUs want more than one (7936 rows of width 256, K and V with
+// the rows around them: 47 / 41 / 41 / 45 us at 256 / 512 / 768 / 1024).
+constexpr int kWideGroups = 512;
+
 // Checks a reconstruction and fills its kernel parameters; `segs` > 0 when it
-// takes the streaming kernel (latent width kw <= 64), whose workgroup count is
-// B * Hkv * segs.
+// takes the streaming kernel (latent width kw <= 64) or the wide one
+// (kw >= 128), whose workgroup count is B * Hkv * segs.
 int prepare_recon(const slimkv_reconstruct_args* a, ReconParams* out, int* segs, int* kw_out) {
     if (!a) return fail(SLIMKV_EINVAL, "null pointer");
     if (a->batch <= 0 || a->rows < 0 || a->rank <= 0 || a->kv_heads <= 0 || a->head_dim != 128)
@@ -257,15 +501,29 @@ int prepare_recon(const slimkv_reconstruct_args* a, ReconParams* out, int* segs,
     p.positions = a->positions; p.pos_sb = a->pos_sb;
     p.B = (int)a->batch; p.n = (int)a->rows; p.R = (int)a->rank; p.Hkv = (int)a->kv_heads;
     p.blockdiag = bd ? 1 : 0; p.k_lo_step = (int)kw;
+    p.in16 = pal16(a->latent) && pal16(a->weight) && al8(a->l_sb) && al8(a->l_sn) && al8(a->rank);
+    p.out16 = pal16(a->out) && al8(a->o_sb) && al8(a->o_sn) && al8(a->o_sh);
     *kw_out = (int)kw;
-    const bool tables16 = !a->positions || (((reinterpret_cast<uintptr_t>(a->cos) | reinterpret_cast<uintptr_t>(a->sin)) & 15) == 0);
-    if (kw <= 64 && tables16) {
+    p.tables16 = !a->positions || (((reinterpret_cast<uintptr_t>(a->cos) | reinterpret_cast<uintptr_t>(a->sin)) & 15) == 0);
+    if (kw <= 64 && p.tables16) {
         // streaming kernel: about 1024 workgroups, each wavefront at least one tile
         const int row_tiles = (p.n + 15) / 16;
         const int64_t heads = (int64_t)p.B * p.Hkv;
         const int sg = (int)std::max<int64_t>(1, std::min<int64_t>((row_tiles + kReconWaves - 1) / kReconWaves,
                                                                    (1024 + heads - 1) / heads));
         if ((int64_t)p.B * p.Hkv * sg > 0x3fffffff) return fail(SLIMKV_EINVAL, "reconstruction grid too large");
+        *segs = sg;
+    } else if (kw >= 128) {
+        // wide kernel: tiles of 32 rows, of 16 where 32 would leave CUs idle;
+        // (and where W of width 512 and the RoPE pieces leave no registers for
+        // the second group: it spilled); row segments in eights where there
+        // are that many (its XCD order)
+        const int64_t heads = (int64_t)p.B * p.Hkv;
+        p.row_frags = heads * ((p.n + 31) / 32) < kWideGroups / 2 || (kw == 512 && a->positions) ? 1 : 2;
+        const int row_tiles = (p.n + 16 * p.row_frags - 1) / (16 * p.row_frags);
+        int sg = (int)std::max<int64_t>(1, std::min<int64_t>(row_tiles, (kWideGroups + heads - 1) / heads));
+        if (sg >= 8) sg = sg / 8 * 8;
+        if (heads * sg > 0x3fffffff) return fail(SLIMKV_EINVAL, "reconstruction grid too large");
         *segs = sg;
     }
     return SLIMKV_OK;
@@ -278,7 +536,13 @@ int launch_prepared(const ReconParams& p, int segs, int kw, hipStream_t st) {
             case 1: e = launch_stream<1>(p, segs, st); break;
             case 2: e = launch_stream<2>(p, segs, st); break;
             case 3: e = launch_stream<3>(p, segs, st); break;
-            default: e = launch_stream<4>(p, segs, st); break;
+            case 4: e = launch_stream<4>(p, segs, st); break;
+            case 8: e = launch_wide<4>(p, segs, st); break;
+            case 12: e = launch_wide<6>(p, segs, st); break;
+            case 16: e = launch_wide<8>(p, segs, st); break;
+            case 24: e = launch_wide<12>(p, segs, st); break;
+            case 32: e = launch_wide<16>(p, segs, st); break;
+            default: return fail(SLIMKV_EUNSUP, "latent width not instantiated");
         }
         return check_hip(e, "reconstruction kernel launch");
     }
@@ -289,11 +553,6 @@ int launch_prepared(const ReconParams& p, int segs, int kw, hipStream_t st) {
         case 2: e = launch_recon<2>(p, grid, st); break;
         case 3: e = launch_recon<3>(p, grid, st); break;
         case 4: e = launch_recon<4>(p, grid, st); break;
-        case 8: e = launch_recon<8>(p, grid, st); break;
-        case 12: e = launch_recon<12>(p, grid, st); break;
-        case 16: e = launch_recon<16>(p, grid, st); break;
-        case 24: e = launch_recon<24>(p, grid, st); break;
-        case 32: e = launch_recon<32>(p, grid, st); break;
         default: return fail(SLIMKV_EUNSUP, "latent width not instantiated");
     }
     return check_hip(e, "reconstruction kernel launch");
@@ -305,6 +564,18 @@ hipError_t launch_stream_pair(const ReconParams& p0, int segs0, const ReconParam
     const int blocks1 = p1.B * p1.Hkv * segs1;
     hipLaunchKernelGGL((recon_stream_pair_kernel<K>), dim3(blocks0 + blocks1), dim3(kReconWaves * 64), 0, st, p0, p1,
                        segs0, segs1, blocks0);
+    return hipGetLastError();
+}
+
+template <int KS>
+hipError_t launch_wide_pair(const ReconParams& p0, int segs0, const ReconParams& p1, int segs1, hipStream_t st) {
+    const int blocks0 = p0.B * p0.Hkv * segs0;
+    const int blocks1 = p1.B * p1.Hkv * segs1;
+    const dim3 grid(blocks0 + blocks1), block(kReconWaves * 64);
+    if (p0.row_frags == 1)
+        hipLaunchKernelGGL((recon_wide_pair_kernel<KS, 1>), grid, block, 0, st, p0, p1, segs0, segs1, blocks0);
+    else
+        hipLaunchKernelGGL((recon_wide_pair_kernel<KS, 2>), grid, block, 0, st, p0, p1, segs0, segs1, blocks0);
     return hipGetLastError();
 }
 
@@ -325,13 +596,22 @@ int reconstruct_pair(const slimkv_reconstruct_args* a, const slimkv_reconstruct_
     if (rc != SLIMKV_OK) return rc;
     if (a->rows == 0) return b->rows == 0 ? SLIMKV_OK : launch_prepared(pb, sb, kb, st);
     if (b->rows == 0) return launch_prepared(pa, sa, ka, st);
-    if (sa > 0 && sb > 0 && ka == kb) {
+    // wide widths share a launch without RoPE and with 16-byte rows
+    const bool pairable =
+        ka <= 64 || (!pa.positions && !pb.positions && pa.in16 && pb.in16 && pa.row_frags == pb.row_frags);
+    if (sa > 0 && sb > 0 && ka == kb && pairable) {
         hipError_t e;
         switch (ka / 16) {
             case 1: e = launch_stream_pair<1>(pa, sa, pb, sb, st); break;
             case 2: e = launch_stream_pair<2>(pa, sa, pb, sb, st); break;
             case 3: e = launch_stream_pair<3>(pa, sa, pb, sb, st); break;
-            default: e = launch_stream_pair<4>(pa, sa, pb, sb, st); break;
+            case 4: e = launch_stream_pair<4>(pa, sa, pb, sb, st); break;
+            case 8: e = launch_wide_pair<4>(pa, sa, pb, sb, st); break;
+            case 12: e = launch_wide_pair<6>(pa, sa, pb, sb, st); break;
+            case 16: e = launch_wide_pair<8>(pa, sa, pb, sb, st); break;
+            case 24: e = launch_wide_pair<12>(pa, sa, pb, sb, st); break;
+            case 32: e = launch_wide_pair<16>(pa, sa, pb, sb, st); break;
+            default: return fail(SLIMKV_EUNSUP, "latent width not instantiated");
         }
         return check_hip(e, "reconstruction pair launch");
     }

@@ -1,0 +1,66 @@
+"""The reconstruction at contracted widths of 128 and more (coupled bases): the
+tile and segment edges of its workgroups, rows off a 16-byte boundary, the RoPE
+epilogue with tables off one, and two problems in one launch."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import attention as oa
+from oracle import rope as orope
+from slimkv_amd.workloads import rope_tables
+from tests.helpers import neighbour_of_exact, to_np
+
+pytestmark = pytest.mark.gpu
+
+D, HKV = 128, 8
+
+
+def _inputs(device, B, n, R, shift):
+    """Latent rows and W starting `shift` elements past a 16-byte boundary."""
+    gen = torch.Generator(device=device).manual_seed(R + n)
+
+    def take(*shape):
+        size = int(np.prod(shape))
+        flat = torch.randn(size + shift, generator=gen, device=device).to(torch.bfloat16)
+        return flat[shift:].view(*shape)
+    lat, w = take(B, n, R), take(HKV * D, R)
+    return lat, w / 16 if not shift else w, torch.randn(HKV * D, generator=gen, device=device).to(torch.bfloat16)
+
+
+@pytest.mark.parametrize('R,B,n,shift', [(128, 1, 1, 0), (192, 2, 17, 0), (256, 1, 33, 4), (384, 3, 1100, 0),
+                                         (512, 1, 40, 0), (512, 2, 1025, 4), (192, 1, 16, 4)])
+def test_wide_reconstruction(device, R, B, n, shift):
+    from slimkv_amd import kernels
+    lat, w, bias = _inputs(device, B, n, R, shift)
+    plain = kernels.reconstruct(lat, w, bias, kv_heads=HKV)
+    exact = oa.reconstruct(to_np(lat)[:, None], to_np(w), to_np(bias), HKV, D, bf16_boundaries=False)
+    rounded = oa.reconstruct(to_np(lat)[:, None], to_np(w), to_np(bias), HKV, D)
+    terms = oa.reconstruct(np.abs(to_np(lat))[:, None], np.abs(to_np(w)), None, HKV, D, bf16_boundaries=False)
+    neighbour_of_exact(to_np(plain).transpose(0, 2, 1, 3), exact, rounded, terms)
+
+    # RoPE and scatter: the reference's bf16 steps on the rows rebuilt above,
+    # the tables one float past a 16-byte boundary where the rows are too
+    off = 1 if shift else 0
+    tables = [torch.empty(2000 * D + off, device=device)[off:].view(2000, D) for _ in range(2)]
+    for t, src in zip(tables, rope_tables(2000, D, 500000.0, device)):
+        t.copy_(src)
+    cos, sin = tables
+    gen = torch.Generator(device=device).manual_seed(5)
+    pos = torch.randint(0, 2000, (B, n), generator=gen, device=device)
+    dst = torch.randperm(n + 3, generator=torch.Generator().manual_seed(3))[:n].to(device)
+    out = torch.zeros(B, HKV, n + 3, D, dtype=torch.bfloat16, device=device).transpose(1, 2)
+    kernels.reconstruct(lat, w, bias, kv_heads=HKV, out=out, dst_rows=dst, positions=pos, cos=cos, sin=sin)
+    c, s, p = to_np(cos).astype(np.float32), to_np(sin).astype(np.float32), pos.cpu().numpy()
+    x = to_np(plain).astype(np.float32)
+    rot = np.stack([orope.rotate_bf16(x[b], c[p[b]][:, None], s[p[b]][:, None]) for b in range(B)])
+    np.testing.assert_array_equal(to_np(out)[:, dst.cpu().numpy()], rot)
+    untouched = np.setdiff1d(np.arange(n + 3), dst.cpu().numpy())
+    assert (to_np(out)[:, untouched] == 0).all()
+
+
+@pytest.mark.parametrize('rows', [(16, 16), (300, 40), (2100, 2100)])
+def test_wide_pair_equals_single_launches(device, rows):
+    from slimkv_amd import kernels
+    problems = [dict(zip(('latent', 'weight', 'bias'), _inputs(device, 1, n, 256, 0)), kv_heads=HKV) for n in rows]
+    for got, kw in zip(kernels.reconstruct_pair(*problems), problems):
+        assert torch.equal(got, kernels.reconstruct(**kw))

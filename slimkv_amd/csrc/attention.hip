@@ -1475,28 +1475,6 @@ struct CombineParams {
 
 constexpr int kMaxSplits = 256;
 constexpr int kMaxLatW = 1024;
-constexpr int kCombineThreads = 128;
-
-__device__ __forceinline__ float block_max128(float v, float* red) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, shfl_xor_f(v, o));
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-    __syncthreads();
-    v = fmaxf(red[0], red[1]);
-    __syncthreads();
-    return v;
-}
-
-__device__ __forceinline__ float block_sum128(float v, float* red) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += shfl_xor_f(v, o);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-    __syncthreads();
-    v = red[0] + red[1];
-    __syncthreads();
-    return v;
-}
-
 // Latent splits written for batch entry b (all of them unless the schedule was compact).
 __device__ __forceinline__ int live_b_splits(const CombineParams& cp, int b) {
     if (!cp.b_len || !cp.b_splits) return cp.b_splits;
@@ -1506,12 +1484,31 @@ __device__ __forceinline__ int live_b_splits(const CombineParams& cp, int b) {
 }
 
 // One workgroup per (b, query head, query): LSE-merge the split partials of
-// both segments, lift the latent accumulator through U_V, fold the biases.
-__global__ void __launch_bounds__(kCombineThreads)
+// both segments, lift the latent accumulator through U_V, fold the biases --
+// for every shape the two narrower kernels below do not take (latents of all
+// KV heads, rebuilt full-width rows, plain attention at any width).  It is
+// bound by memory round trips, so the loads that depend on nothing are issued
+// first (U_V pieces, the first partials of each segment, one split's
+// statistics a thread) and the rest by 1024 threads side by side: a thread
+// owns one four-column quad of every T / quads-th split, and eight
+// neighbouring lanes share a row of U_V, reading its pieces as whole cache
+// lines.  A serial loop over splits and U_V columns on 128 threads took
+// 46.5 us for 32 rows of 256 latent splits of width 256 (one sequence, now
+// 10.0), 12.7 for 256 rows of 32 splits (7.4) and 13.9 for 64 rows over
+// rebuilt rows (6.8); 512 threads with twice the loads ahead the same.
+constexpr int kWideThreads = 1024;
+constexpr int kWideLift = 6;         // U_V pieces a lane: latent widths up to 384
+constexpr int kWideAhead = 4;        // latent quads a thread issues before the statistics (raw: half)
+
+__global__ void __launch_bounds__(kWideThreads)
 combine_kernel(CombineParams cp) {
+    constexpr int T = kWideThreads, NW = T / 64;
     __shared__ float wts[2 * kMaxSplits];
+    __shared__ float4 part[2][T];            // quad sums of the latent and the raw segment by split group
     __shared__ float accb[kMaxLatW];
-    __shared__ float red[2];
+    __shared__ float acca[512];
+    __shared__ float red[3][NW];
+    const int t = threadIdx.x;
     const int HL = cp.Hq * cp.Lq;
     const int pr = blockIdx.x % HL;
     const int b = blockIdx.x / HL;
@@ -1521,87 +1518,148 @@ combine_kernel(CombineParams cp) {
     const int64_t row = (int64_t)b * HL + pr;
     const float* aml = cp.a_ml + row * cp.a_splits * 2;
     const float* bml = cp.b_splits ? cp.b_ml + row * cp.b_splits * 2 : nullptr;
-    const float shift = (cp.b_splits && cp.b_shift) ? cp.b_shift[row] * kLog2e : 0.f;
     const int bsp = live_b_splits(cp, b);
     const int total = cp.a_splits + bsp;
+    const bool lift = cp.b_splits && cp.up_v;
 
-    // Split maxima and masses, one split per thread.
-    float mloc = kNegInf;
-    for (int s = threadIdx.x; s < total; s += kCombineThreads) {
-        float mv = s < cp.a_splits ? aml[2 * s] : bml[2 * (s - cp.a_splits)];
-        if (s >= cp.a_splits && mv != kNegInf) mv += shift;
-        wts[s] = mv;
-        mloc = fmaxf(mloc, mv);
+    // Loads that depend on nothing.  Out-of-range ones read the operand's
+    // first element instead and are dropped where they would be used.
+    const int aq = cp.a_w / 4, bq = cp.b_splits ? cp.b_w / 4 : 1;
+    const int ga = T / aq, gb = T / bq;                     // split groups
+    const int ka = t % aq, sa = t / aq, kb = t % bq, sb = t / bq;
+    const float4* aacc = reinterpret_cast<const float4*>(cp.a_acc + row * cp.a_splits * cp.a_w);
+    const float4* bacc = reinterpret_cast<const float4*>(cp.b_splits ? cp.b_acc + row * cp.b_splits * cp.b_w : cp.a_acc);
+    const bool ina = sa < ga, inb = cp.b_splits && sb < gb;
+    float4 fa[kWideAhead / 2], fb[kWideAhead];
+#pragma unroll
+    for (int i = 0; i < kWideAhead / 2; ++i) {
+        const int sp = sa + i * ga;
+        fa[i] = aacc[ina && sp < cp.a_splits ? sp * aq + ka : 0];
     }
-    const float M = block_max128(mloc, red);
+#pragma unroll
+    for (int i = 0; i < kWideAhead; ++i) {
+        const int sp = sb + i * gb;
+        fb[i] = bacc[inb && sp < bsp ? sp * bq + kb : 0];
+    }
+    const int d8 = t / 8, piece = t % 8;                    // output d8 (T / 8 = 128 at a time)
+    u32x4 w[kWideLift];
+    const uint16_t* wrow = lift ? cp.up_v + (cp.blockdiag ? h * cp.b_w : 0) : nullptr;
+    auto lift_load = [&](int d) {
+        const uint16_t* src = wrow + ((int64_t)h * cp.D + d) * cp.up_v_ld;
+#pragma unroll
+        for (int i = 0; i < kWideLift; ++i) {
+            const int k = 8 * (piece + 8 * i);
+            w[i] = *reinterpret_cast<const u32x4*>(src + (k < cp.b_w ? k : 0));
+        }
+    };
+    if (lift) lift_load(min(d8, cp.D - 1));
+    const float shift = (cp.b_splits && cp.b_shift) ? cp.b_shift[row] * kLog2e : 0.f;
+
+    // Split maxima and masses: at most 2 * kMaxSplits <= T splits, one a thread.
+    float mv = kNegInf, lv = 0.f;
+    if (t < cp.a_splits) {
+        mv = aml[2 * t];
+        lv = aml[2 * t + 1];
+    } else if (t < total) {
+        mv = bml[2 * (t - cp.a_splits)];
+        lv = bml[2 * (t - cp.a_splits) + 1];
+        if (mv != kNegInf) mv += shift;
+    }
+    auto wave_reduce = [](float v, auto op) {
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) v = op(v, shfl_xor_f(v, o));
+        return v;
+    };
+    auto maxf = [](float x, float y) { return fmaxf(x, y); };
+    auto addf = [](float x, float y) { return x + y; };
+    const int lane = t & 63, wave = t >> 6;
+    const float wm = wave_reduce(mv, maxf);
+    if (lane == 0) red[0][wave] = wm;
+    __syncthreads();
+    const float M = wave_reduce(lane < NW ? red[0][lane] : kNegInf, maxf);
     const float Mref = M == kNegInf ? 0.f : M;
-    float la = 0.f, lb = 0.f;
-    for (int s = threadIdx.x; s < total; s += kCombineThreads) {
-        const float wgt = wts[s] == kNegInf ? 0.f : fast_exp2(wts[s] - Mref);
-        wts[s] = wgt;
-        if (s < cp.a_splits) la += aml[2 * s + 1] * wgt;
-        else lb += bml[2 * (s - cp.a_splits) + 1] * wgt;
+    const float wgt = mv == kNegInf ? 0.f : fast_exp2(mv - Mref);
+    if (t < total) wts[t] = wgt;
+    const float la = wave_reduce(t < cp.a_splits ? lv * wgt : 0.f, addf);
+    const float lb = wave_reduce(t >= cp.a_splits ? lv * wgt : 0.f, addf);
+    if (lane == 0) {
+        red[1][wave] = la;
+        red[2][wave] = lb;
     }
-    const float LA = block_sum128(la, red);
-    const float LB = block_sum128(lb, red);
+    __syncthreads();
+    const float LA = wave_reduce(lane < NW ? red[1][lane] : 0.f, addf);
+    const float LB = wave_reduce(lane < NW ? red[2][lane] : 0.f, addf);
     const float L = LA + LB;
 
-    if (cp.b_splits) {
-        // Weighted latent accumulator: threads split (k, split group).
-        const float* bacc = cp.b_acc + row * cp.b_splits * cp.b_w;
-        const float* wb = wts + cp.a_splits;
-        if (cp.b_w <= kCombineThreads / 2) {
-            const int groups = kCombineThreads / cp.b_w;
-            const int k = threadIdx.x % cp.b_w, gsel = threadIdx.x / cp.b_w;
-            float sum = 0.f;
-            if (gsel < groups)
-                for (int s = gsel; s < bsp; s += groups) sum += bacc[(int64_t)s * cp.b_w + k] * wb[s];
-            __shared__ float part[kCombineThreads];
-            part[threadIdx.x] = sum;
-            __syncthreads();
-            if (threadIdx.x < cp.b_w) {
-                float t = 0.f;
-                for (int g2 = 0; g2 < groups; ++g2) t += part[g2 * cp.b_w + threadIdx.x];
-                accb[threadIdx.x] = t;
-            }
-        } else {
-            for (int k = threadIdx.x; k < cp.b_w; k += kCombineThreads) {
-                float sum = 0.f;
-                for (int s = 0; s < bsp; ++s) sum += bacc[(int64_t)s * cp.b_w + k] * wb[s];
-                accb[k] = sum;
-            }
-        }
-        __syncthreads();
-    }
-    const float inv = L > 0.f ? 1.f / L : 0.f;
-    const float* aacc = cp.a_acc + row * cp.a_splits * cp.a_w;
-    uint16_t* orow = cp.out + (int64_t)b * cp.o_sb + (int64_t)lq * cp.o_sl + (int64_t)j * cp.o_sh;
-    for (int dd = threadIdx.x; dd < cp.D; dd += kCombineThreads) {
-        float sum = 0.f;
-        for (int s = 0; s < cp.a_splits; ++s) sum += aacc[(int64_t)s * cp.a_w + dd] * wts[s];
-        if (cp.b_splits && !cp.up_v) {
-            sum += accb[dd];          // full-dim second segment: no lift
-        } else if (cp.b_splits) {
-            const int64_t wrow = (int64_t)h * cp.D + dd;
-            const uint16_t* wr = cp.up_v + wrow * cp.up_v_ld + (cp.blockdiag ? h * cp.b_w : 0);
-            float lift = 0.f;
-            for (int k = 0; k < cp.b_w; k += 8) {
-                const u32x4 wv = *reinterpret_cast<const u32x4*>(wr + k);
-                const uint32_t ws[4] = {wv.x, wv.y, wv.z, wv.w};
+    // Weighted quad sums of the thread's splits, then over the split groups.
+    auto fma4 = [](float4& acc, const float4& x, float s) {
+        acc.x = fmaf(x.x, s, acc.x);
+        acc.y = fmaf(x.y, s, acc.y);
+        acc.z = fmaf(x.z, s, acc.z);
+        acc.w = fmaf(x.w, s, acc.w);
+    };
+    float4 qa = make_float4(0.f, 0.f, 0.f, 0.f), qb = qa;
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    lift += bf16_to_f32(ws[e] & 0xffffu) * accb[k + 2 * e];
-                    lift += bf16_to_f32(ws[e] >> 16) * accb[k + 2 * e + 1];
+    for (int i = 0; i < kWideAhead / 2; ++i)
+        if (ina && sa + i * ga < cp.a_splits) fma4(qa, fa[i], wts[sa + i * ga]);
+#pragma unroll
+    for (int i = 0; i < kWideAhead; ++i)
+        if (inb && sb + i * gb < bsp) fma4(qb, fb[i], wts[cp.a_splits + sb + i * gb]);
+    if (ina)
+#pragma unroll 4
+        for (int sp = sa + kWideAhead / 2 * ga; sp < cp.a_splits; sp += ga) fma4(qa, aacc[sp * aq + ka], wts[sp]);
+    if (inb)
+#pragma unroll 4
+        for (int sp = sb + kWideAhead * gb; sp < bsp; sp += gb) fma4(qb, bacc[sp * bq + kb], wts[cp.a_splits + sp]);
+    part[0][t] = qb;
+    part[1][t] = qa;
+    __syncthreads();
+    const int bw = cp.b_splits ? cp.b_w : 0;
+    for (int k = t; k < bw + cp.a_w; k += T) {
+        const bool latent = k < bw;
+        const int c = latent ? k : k - bw, quads = latent ? bq : aq, groups = latent ? gb : ga;
+        const float* src = reinterpret_cast<const float*>(part[latent ? 0 : 1]) + c;
+        float sum = 0.f;
+#pragma unroll 4
+        for (int g2 = 0; g2 < groups; ++g2) sum += src[4 * g2 * quads];
+        (latent ? accb : acca)[c] = sum;
+    }
+    __syncthreads();
+
+    const float inv = L > 0.f ? 1.f / L : 0.f;
+    uint16_t* orow = cp.out + (int64_t)b * cp.o_sb + (int64_t)lq * cp.o_sl + (int64_t)j * cp.o_sh;
+    if (lift) {
+        for (int d = d8; d < cp.D; d += T / 8) {            // eight lanes a row stay together
+            if (d != d8) lift_load(d);
+            float sum = 0.f;
+#pragma unroll
+            for (int i = 0; i < kWideLift; ++i) {
+                const int k = 8 * (piece + 8 * i);
+                if (k < cp.b_w) {
+                    const float4 x0 = *reinterpret_cast<const float4*>(accb + k);
+                    const float4 x1 = *reinterpret_cast<const float4*>(accb + k + 4);
+                    sum += lo_bf16(w[i].x) * x0.x + hi_bf16(w[i].x) * x0.y;
+                    sum += lo_bf16(w[i].y) * x0.z + hi_bf16(w[i].y) * x0.w;
+                    sum += lo_bf16(w[i].z) * x1.x + hi_bf16(w[i].z) * x1.y;
+                    sum += lo_bf16(w[i].w) * x1.z + hi_bf16(w[i].w) * x1.w;
                 }
             }
-            sum += lift;
-            if (cp.up_v_bias) sum += bf16_to_f32(cp.up_v_bias[wrow]) * LB;
+#pragma unroll
+            for (int o = 4; o > 0; o >>= 1) sum += shfl_xor_f(sum, o);
+            if (piece == 0) {
+                sum += acca[d];
+                if (cp.up_v_bias) sum += bf16_to_f32(cp.up_v_bias[(int64_t)h * cp.D + d]) * LB;
+                orow[d] = (uint16_t)pack_bf16(sum * inv, 0.f);
+            }
         }
-        orow[dd] = (uint16_t)pack_bf16(sum * inv, 0.f);
+    } else {
+        for (int d = t; d < cp.D; d += T) {
+            const float sum = acca[d] + (cp.b_splits ? accb[d] : 0.f);   // full-width second segment: no lift
+            orow[d] = (uint16_t)pack_bf16(sum * inv, 0.f);
+        }
     }
-    if (cp.lse && threadIdx.x == 0) {
+    if (cp.lse && t == 0)
         cp.lse[((int64_t)b * cp.Hq + j) * cp.Lq + lq] = L > 0.f ? (M + __log2f(L)) * kLn2 : kNegInf;
-    }
 }
 
 // Raw buffer resource over `bytes` bytes at p (a null p with 0 bytes: every
@@ -2003,7 +2061,7 @@ void launch_combine(const CombineParams& cp, int rows, hipStream_t st) {
     else if (combine_fast_ok(cp, 256))
         hipLaunchKernelGGL(combine_fast_kernel<256>, dim3(rows), dim3(256), 0, st, cp);
     else
-        hipLaunchKernelGGL(combine_kernel, dim3(rows), dim3(kCombineThreads), 0, st, cp);
+        hipLaunchKernelGGL(combine_kernel, dim3(rows), dim3(kWideThreads), 0, st, cp);
 }
 
 // ---------------------------------------------------------------------------

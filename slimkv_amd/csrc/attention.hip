@@ -551,7 +551,7 @@ __device__ __forceinline__ float kbias_dot(const u32x4 (&q)[4], const u32x4 (&bk
 // never exchange data, and write their own partials.
 // PAGED: 0 dense rows, 1 rows through per-lane page ids, 2 rows through the
 // tile's two pages (pages of at least 16 rows).
-template <int KS, int DEPTH, int PAGED = 0, int SEG2 = 0, int RAWPG = 0, int FQ = 0>
+template <int KS, int DEPTH, int PAGED = 0, int SEG2 = 0, int RAWPG = 0, int FQ = 0, int NW = kWaves>
 __device__ __forceinline__ void split_segment(const Seg& sg, int w, int B, int Lq, int Hq,
                                               float scale_log2, char* lds, const SegRows2* two = nullptr,
                                               const RawPagesArg* rawp = nullptr, const QRope* qr = nullptr,
@@ -568,12 +568,12 @@ __device__ __forceinline__ void split_segment(const Seg& sg, int w, int B, int L
     const int col = lane & 15;
     const int grp = lane >> 4;
 
-    // Wave items: (batch, split, slot) with the slot fastest, kWaves per
-    // workgroup -- the waves of a workgroup read the same key rows (different
+    // Wave items: (batch, split, slot) with the slot fastest, NW (the
+    // workgroup's waves) per workgroup -- the waves of a workgroup read the same key rows (different
     // heads) of one split, or of consecutive splits when a split has fewer
     // slots than the workgroup has waves.
     const int slots = sg.hk * sg.tiles;
-    const int64_t item = (int64_t)w * kWaves + wave;
+    const int64_t item = (int64_t)w * NW + wave;
     const int slot = (int)(item % slots);
     const int64_t split_item = item / slots;
     int s, b;
@@ -1022,6 +1022,12 @@ split_kernel(SplitParams prm) {
                                                                  lds, &prm.two, nullptr, FQ ? &prm.qrope : nullptr,
                                                                  FQ ? &prm.absorb : nullptr);
 }
+
+}  // namespace slimkv
+
+#include "coupled.hpp"
+
+namespace slimkv {
 
 // ---------------------------------------------------------------------------
 // fused reconstruction decode: beacon K rebuilt and rotated per 16-key tile
@@ -2352,10 +2358,10 @@ struct SegPlan {
     int tiles, cols, splits, rows_per_split, nwg, wown, ks;
 };
 
-// Workgroups covering B * splits * slots wave items, kWaves per workgroup.
-int wave_item_groups(int B, int splits, int slots) {
+// Workgroups covering B * splits * slots wave items, `waves` per workgroup.
+int wave_item_groups(int B, int splits, int slots, int waves = kWaves) {
     const int64_t items = (int64_t)B * splits * slots;
-    return (int)((items + kWaves - 1) / kWaves);
+    return (int)((items + waves - 1) / waves);
 }
 
 // Split the key range so the launch holds a few workgroups per CU.
@@ -2586,6 +2592,8 @@ namespace {
 
 struct LatentPlan {
     SegPlan raw, lat;
+    int coupled;          // latent rows by the coupled kernel: groups of 16 query rows a workgroup, 0 = split kernel
+    int groups;           // workgroups that share a sequence's query rows there
     int wq;               // q_lat width per head
     int parts;
     size_t qrot_off, qlat_off, shift_off, rml_off, racc_off, lml_off, lacc_off, total;
@@ -2757,6 +2765,22 @@ int plan_latent(const slimkv_latent_decode_args* a, LatentPlan* p, const PagedRo
     if (lat_req <= 0 && !pg)
         lat_req = (int)std::max<int64_t>(1, std::min<int64_t>(kMaxSplits, (int64_t)lat_target * kWaves / lat_tiles));
     p->lat = plan_segment((int)B, 1, P, cols, (int)nl, span, rv, lat_req, lat_target);
+    p->coupled = 0;
+    if (!bd && !pg && has_lat) {
+        // Coupled bases: workgroups that hold every query row (up to 80) and
+        // one such workgroup a CU.  More than one a CU only adds partials;
+        // fewer splits than tiles of 64 rows keep the merge short.
+        const int rows16 = (P + 15) / 16;
+        p->groups = (rows16 + 4) / 5;
+        p->coupled = std::max(2, (rows16 + p->groups - 1) / p->groups);
+        const int tiles = (int)((nl + kTileKeys - 1) / kTileKeys);
+        int splits = a->lat_splits;
+        if (splits <= 0) splits = (int)std::max<int64_t>(1, cu / ((int64_t)B * p->groups));
+        splits = std::min({splits, tiles, kMaxSplits});
+        p->lat.splits = splits;
+        p->lat.rows_per_split = 0;
+        p->lat.nwg = (int)B * splits * p->groups;
+    }
     if (pg && a->lat_splits <= 0) {
         // Compact schedule: size the splits from the total row count so the
         // non-empty splits of all sequences make about fill_target items.
@@ -2775,6 +2799,7 @@ int plan_latent(const slimkv_latent_decode_args* a, LatentPlan* p, const PagedRo
     // before the latent ones.
     p->raw = plan_segment((int)B, (int)Hkv, (int)Lq * g, 16, (int)a->raw_keys, (int)D, (int)D, raw_req0, 0);
     if (p->raw.tiles != 1 || p->raw.ks != 8) return fail(SLIMKV_EUNSUP, "raw tile shape");
+    if (p->coupled) p->raw.nwg = wave_item_groups((int)B, p->raw.splits, (int)Hkv, kCoupledWaves);
     p->wq = rk;
     int parts = 1;
     while (parts < 16 && g * (int)Lq * (p->wq / 8) * parts * 2 <= 256) parts *= 2;
@@ -2939,7 +2964,22 @@ int latent_decode_run(const slimkv_latent_decode_args* a, const PagedRows* pg, v
     const bool paged = pg && has_lat;
     if (paged && ka > 8) return fail(SLIMKV_EUNSUP, "paged decode handles latent tiles up to 128 wide");
     const int grid = prm.seg[0].nwg + (has_lat ? prm.seg[1].nwg : 0);
-    if (stages & SLIMKV_STAGE_ATTEND) {
+    if ((stages & SLIMKV_STAGE_ATTEND) && p.coupled) {
+        const Seg& l = prm.seg[0];
+        CoupledParams cq{};
+        cq.q = q_lat;
+        cq.k = CoupledRows{l.k, l.k_sb, l.k_sn, prm.two.k2, prm.two.k2_sb, prm.two.k2_sn, Rk};
+        cq.v = CoupledRows{l.v, l.v_sb, l.v_sn, prm.two.v2, prm.two.v2_sb, prm.two.v2_sn, Rv};
+        cq.n = l.n;
+        cq.n1 = a->lat_k2 ? prm.two.n1 : l.n;
+        cq.seqlens = l.seqlens;
+        cq.causal = l.causal; cq.splits = l.splits; cq.groups = p.groups;
+        cq.part_ml = l.part_ml; cq.part_acc = l.part_acc;
+        cq.B = B; cq.Lq = Lq; cq.Hq = Hq; cq.nwg = l.nwg;
+        cq.scale_log2 = prm.scale_log2;
+        rc = check_hip(launch_coupled(p.coupled, cq, r, st), "coupled kernel launch");
+        if (rc != SLIMKV_OK) return rc;
+    } else if (stages & SLIMKV_STAGE_ATTEND) {
         const bool seg2 = has_lat && a->lat_k2 != nullptr;
         rc = check_hip(fused ? launch_split_fused(ka, prm, grid, st, paged, seg2)
                              : launch_split_any(ka, kb, prm, grid, st, paged, seg2),
@@ -3027,6 +3067,14 @@ extern "C" int slimkv_latent_decode_noalloc(const slimkv_latent_decode_args* a, 
     LatentPlan p{};
     int rc = plan_latent(a, &p);
     if (rc != SLIMKV_OK) return rc;
+    // Coupled bases plan a workgroup a CU, up to 80 query rows each: fewer
+    // splits where their partials would not fit.
+    slimkv_latent_decode_args fit = *a;
+    while (p.coupled && p.total > (size_t)SLIMKV_NOALLOC_SCRATCH_BYTES && p.lat.splits > 1) {
+        fit.lat_splits = p.lat.splits / 2;
+        rc = plan_latent(&fit, &p);
+        if (rc != SLIMKV_OK) return rc;
+    }
     if (p.total > (size_t)SLIMKV_NOALLOC_SCRATCH_BYTES)
         return fail(SLIMKV_EWORKSPACE, "slimkv_latent_decode_noalloc: this call needs " + std::to_string(p.total) +
                                            " bytes of workspace, more than the " +
@@ -3035,7 +3083,7 @@ extern "C" int slimkv_latent_decode_noalloc(const slimkv_latent_decode_args* a, 
     void* ws = nullptr;
     rc = scratch_address(&ws);
     if (rc != SLIMKV_OK) return rc;
-    return latent_decode_run(a, nullptr, ws, (size_t)SLIMKV_NOALLOC_SCRATCH_BYTES, stream);
+    return latent_decode_run(&fit, nullptr, ws, (size_t)SLIMKV_NOALLOC_SCRATCH_BYTES, stream);
 }
 
 extern "C" size_t slimkv_paged_latent_decode_workspace(const slimkv_paged_latent_decode_args* a) {

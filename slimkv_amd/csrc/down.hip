@@ -143,6 +143,135 @@ __global__ void __launch_bounds__(256) down_pair_kernel(DownParams p0, DownParam
     else down_body(p1, blockIdx.x - blocks0);
 }
 
+// Weights without blocks (every latent contracts the whole row, K = the hidden
+// size): a workgroup of eight waves owns TR rows x TR outputs over all of K,
+// each wave an eighth of K, and the waves' sums meet in LDS.  A wave copies its
+// K chunk of the TR x rows and TR W rows to LDS in lane order (whole cache
+// lines, the next chunk in flight meanwhile) and reads the MFMA operands from
+// there; no barrier before the final sum.  Bound by the round trips of a
+// wave's few chunks.  down_kernel reads its operands straight into MFMA lanes
+// (sixteen rows per sixteen lanes: line lookups bound it) and needs a second
+// launch for its split partials: K and V latents (256 + 256) of 256 rows of
+// 4096, 31 us in four launches -> 11.5 in one; of 1024 rows 56 -> 20.
+// Row strides are odd multiples of 16 bytes past a multiple of 128, so eight
+// rows' 16-byte reads meet distinct banks.
+constexpr int kDownWaves = 8;
+
+template <int TR>
+struct DownTile {
+    static constexpr int KC = TR == 32 ? 128 : 64;                     // K elements of a chunk
+    static constexpr int STRIDE = 2 * KC + 16;
+    static constexpr int WAVE_BYTES = 2 * TR * STRIDE;
+    static constexpr int SUM_STRIDE = TR + 4;                          // floats; a row's quads stay 16-byte aligned
+    static constexpr int SUM_BYTES = kDownWaves * TR * SUM_STRIDE * 4;
+    static constexpr int LDS = kDownWaves * WAVE_BYTES > SUM_BYTES ? kDownWaves * WAVE_BYTES : SUM_BYTES;
+};
+
+template <int TR>
+__device__ __forceinline__ void down_tile_body(const DownParams& p, int block, char* lds) {
+    using T = DownTile<TR>;
+    constexpr int F = TR / 16, C = T::KC / 8, PIECES = 2 * TR * C / 64;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int col = lane & 15, grp = lane >> 4;
+    const int M = p.B * p.n;
+    const int ntiles = (p.N + TR - 1) / TR;
+    const int n0 = block % ntiles * TR, m0 = block / ntiles * TR;
+    // the wave's share of K in whole chunks
+    const int chunks = (p.K + T::KC - 1) / T::KC;
+    const int k_lo = wave * chunks / kDownWaves * T::KC, k_hi = min(p.K, (wave + 1) * chunks / kDownWaves * T::KC);
+
+    // piece i of a chunk: row (64 i + lane) / C (x rows, then W rows), 16
+    // bytes at column (64 i + lane) % C; the same column for every piece
+    constexpr int STEP = 64 / C;
+    const int pc = lane % C, pr = lane / C;
+    const uint16_t* src[PIECES];
+#pragma unroll
+    for (int i = 0; i < PIECES; ++i) {
+        const int row = pr + i * STEP;
+        if (i < PIECES / 2) {
+            const int m = min(m0 + row, M - 1);
+            const int b = m / p.n, j = m % p.n;
+            const int64_t r = p.rows ? p.rows[j] : j;
+            src[i] = p.x + (int64_t)b * p.x_sb + (r >= 0 && r < p.length ? r : 0) * p.x_sl + 8 * pc;
+        } else {
+            src[i] = p.w + (int64_t)min(n0 + row - TR, p.N - 1) * p.K + 8 * pc;
+        }
+    }
+    u32x4 stage[PIECES];
+    auto fetch = [&](int k) {
+        const int kk = k + 8 * pc < p.K ? k : -8 * pc;      // pieces past K read the row's first, zeroed below
+#pragma unroll
+        for (int i = 0; i < PIECES; ++i) stage[i] = *reinterpret_cast<const u32x4*>(src[i] + kk);
+    };
+    if (k_lo < k_hi) fetch(k_lo);
+    v4f acc[F][F];
+#pragma unroll
+    for (int a = 0; a < F; ++a)
+#pragma unroll
+        for (int b = 0; b < F; ++b) acc[a][b] = v4f{0.f, 0.f, 0.f, 0.f};
+    char* own = lds + wave * T::WAVE_BYTES;
+    auto fence = [] {                                       // a wave's LDS accesses run in order
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
+    for (int k = k_lo; k < k_hi; k += T::KC) {
+        const bool in = k + 8 * pc < p.K;
+#pragma unroll
+        for (int i = 0; i < PIECES; ++i)
+            *reinterpret_cast<u32x4*>(own + (pr + i * STEP) * T::STRIDE + 16 * pc) = zero_if_not(in, stage[i]);
+        fence();
+        if (k + T::KC < k_hi) fetch(k + T::KC);
+#pragma unroll
+        for (int ks = 0; ks < T::KC / 32; ++ks) {
+            u32x4 x[F], w[F];
+#pragma unroll
+            for (int f = 0; f < F; ++f) {
+                x[f] = *reinterpret_cast<const u32x4*>(own + (16 * f + col) * T::STRIDE + 64 * ks + 16 * grp);
+                w[f] = *reinterpret_cast<const u32x4*>(own + (TR + 16 * f + col) * T::STRIDE + 64 * ks + 16 * grp);
+            }
+#pragma unroll
+            for (int a = 0; a < F; ++a)
+#pragma unroll
+                for (int b = 0; b < F; ++b) acc[a][b] = mfma32(w[a], x[b], acc[a][b]);
+        }
+        fence();
+    }
+    __syncthreads();
+    // lane (row 16 b + col) holds outputs 16 a + 4 grp + [0, 4)
+    float* sums = reinterpret_cast<float*>(lds);
+#pragma unroll
+    for (int a = 0; a < F; ++a)
+#pragma unroll
+        for (int b = 0; b < F; ++b)
+            *reinterpret_cast<v4f*>(sums + (wave * TR + 16 * b + col) * T::SUM_STRIDE + 16 * a + 4 * grp) = acc[a][b];
+    __syncthreads();
+    for (int q = tid; q < TR * TR / 4; q += 64 * kDownWaves) {
+        const int row = q / (TR / 4), nn = q % (TR / 4) * 4;
+        const int m = m0 + row;
+        if (m >= M || n0 + nn >= p.N) continue;
+        v4f sum = *reinterpret_cast<const v4f*>(sums + row * T::SUM_STRIDE + nn);
+#pragma unroll
+        for (int w = 1; w < kDownWaves; ++w)
+            sum += *reinterpret_cast<const v4f*>(sums + (w * TR + row) * T::SUM_STRIDE + nn);
+        const int b = m / p.n, i = m % p.n;
+        const int64_t r = p.rows ? p.rows[i] : i;
+        if (r < 0 || r >= p.length) sum = v4f{0.f, 0.f, 0.f, 0.f};   // a row outside x projects to zeros
+        uint16_t* dst = dst_row(p, b, i);
+        if (dst)
+            *reinterpret_cast<u32x2*>(dst + n0 + nn) = u32x2{pack_bf16(sum[0], sum[1]), pack_bf16(sum[2], sum[3])};
+    }
+}
+
+template <int TR>
+__global__ void __launch_bounds__(64 * kDownWaves) __attribute__((amdgpu_waves_per_eu(2)))
+down_tile_kernel(DownParams p0, DownParams p1, int blocks0) {
+    __shared__ __attribute__((aligned(16))) char lds[DownTile<TR>::LDS];
+    if ((int)blockIdx.x < blocks0) down_tile_body<TR>(p0, blockIdx.x, lds);
+    else down_tile_body<TR>(p1, blockIdx.x - blocks0, lds);
+}
+
 // Sum the split partials in split order and round once to bf16.
 __global__ void __launch_bounds__(256) down_reduce_kernel(DownParams p) {
     const int64_t M = (int64_t)p.B * p.n;
@@ -165,6 +294,7 @@ bool al16(const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15) == 0
 
 struct DownPlan {
     int splits, kchunk;
+    int tile;            // down_tile_kernel's TR, 0: down_kernel
     size_t bytes;
 };
 
@@ -180,6 +310,20 @@ int plan_down(const slimkv_down_project_args* a, DownPlan* plan) {
         (reinterpret_cast<uintptr_t>(a->out) & 7))
         return fail(SLIMKV_EINVAL, "x rows must be 16-byte aligned and out rows 8-byte aligned");
     const int64_t M = a->batch * a->row_count;
+    // Weights without blocks: tiles of 32 while two problems of them (the K and
+    // V latents share a launch) fit the CUs once, a workgroup each, else of 64:
+    // a quarter of the tiles, half the reads (1024 rows of 4096 to 256 + 256
+    // with the rebuild after it: 33.3 us with tiles of 32, 25.7 with 64; 1024
+    // to 384 + 384 28.7 against 28.5; 256 rows, 32: 15.7).
+    plan->tile = 0;
+    plan->splits = 1;
+    plan->kchunk = 0;
+    plan->bytes = 0;
+    if (a->blocks == 1) {
+        const int64_t tiles = (M + 31) / 32 * ((a->out_features + 31) / 32);
+        plan->tile = tiles <= device_cu_count() / 2 ? 32 : 64;
+        return SLIMKV_OK;
+    }
     const int64_t kb = a->in_features / a->blocks;
     const int64_t base = (a->out_features + 63) / 64 * ((M + 63) / 64);
     int splits = 1;
@@ -233,6 +377,20 @@ int64_t down_grid(const DownParams& p) {
     return (p.N + 63) / 64 * ((M + 63) / 64) * p.splits;
 }
 
+int64_t tile_grid(const DownParams& p, int tile) {
+    return ((int64_t)p.B * p.n + tile - 1) / tile * ((p.N + tile - 1) / tile);
+}
+
+int launch_tiles(int tile, const DownParams& p0, const DownParams* p1, hipStream_t st) {
+    const int64_t g0 = tile_grid(p0, tile), g1 = p1 ? tile_grid(*p1, tile) : 0;
+    if (g0 + g1 > 0x7fffffff) return fail(SLIMKV_EINVAL, "down-projection grid too large");
+    const dim3 grid((unsigned)(g0 + g1)), block(64 * kDownWaves);
+    const DownParams& second = p1 ? *p1 : p0;
+    if (tile == 32) hipLaunchKernelGGL(down_tile_kernel<32>, grid, block, 0, st, p0, second, (int)g0);
+    else hipLaunchKernelGGL(down_tile_kernel<64>, grid, block, 0, st, p0, second, (int)g0);
+    return check_hip(hipGetLastError(), "down-projection launch");
+}
+
 int down_run(const slimkv_down_project_args* a, const slimkv_page_rows* pg, void* workspace, size_t workspace_bytes,
              void* stream) {
     DownPlan plan{};
@@ -243,8 +401,9 @@ int down_run(const slimkv_down_project_args* a, const slimkv_page_rows* pg, void
     const int64_t M = a->batch * a->row_count;
     if (M == 0) return SLIMKV_OK;
     const DownParams p = down_params(a, pg, plan, workspace);
-    const int64_t grid = down_grid(p);
     hipStream_t st = static_cast<hipStream_t>(stream);
+    if (plan.tile) return launch_tiles(plan.tile, p, nullptr, st);
+    const int64_t grid = down_grid(p);
     hipLaunchKernelGGL(down_kernel, dim3((unsigned)grid), dim3(256), 0, st, p);
     rc = check_hip(hipGetLastError(), "down-projection launch");
     if (rc != SLIMKV_OK || p.splits == 1) return rc;
@@ -280,14 +439,16 @@ extern "C" int slimkv_down_project_pair(const slimkv_down_project_args* a, const
     if (need && (!workspace || workspace_bytes < need)) return fail(SLIMKV_EWORKSPACE, "workspace too small");
     char* ws = static_cast<char*>(workspace);
     const int64_t Ma = a->batch * a->row_count, Mb = b->batch * b->row_count;
-    if (pa.splits > 1 || pb.splits > 1 || Ma == 0 || Mb == 0) {
-        // split partials (a reduce launch each) or an empty problem: one at a time
+    if (pa.splits > 1 || pb.splits > 1 || pa.tile != pb.tile || Ma == 0 || Mb == 0) {
+        // split partials (a reduce launch each), different kernels or an empty
+        // problem: one at a time
         rc = down_run(a, nullptr, ws, align256(pa.bytes), stream);
         if (rc != SLIMKV_OK) return rc;
         return down_run(b, nullptr, ws ? ws + align256(pa.bytes) : nullptr, pb.bytes, stream);
     }
     const DownParams p0 = down_params(a, nullptr, pa, nullptr);
     const DownParams p1 = down_params(b, nullptr, pb, nullptr);
+    if (pa.tile) return launch_tiles(pa.tile, p0, &p1, static_cast<hipStream_t>(stream));
     const int64_t g0 = down_grid(p0), g1 = down_grid(p1);
     if (g0 + g1 > 0x7fffffff) return fail(SLIMKV_EINVAL, "down-projection grid too large");
     hipLaunchKernelGGL(down_pair_kernel, dim3((unsigned)(g0 + g1)), dim3(256), 0, static_cast<hipStream_t>(stream), p0,

@@ -993,6 +993,9 @@ struct SplitDepth {
 template <int KA, int KB, int PAGED = 0, int SEG2 = 0, int RAWPG = 0, int FQ = 0>
 __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(SplitWaves<KA>::value)))
 split_kernel(SplitParams prm) {
+    // Rows of 128 elements may be head rows: their queries are rotated here
+    // where SplitParams::qrope is given (the reconstruction decode).
+    constexpr bool QR = FQ || (KA == 8 && !PAGED && !SEG2);
     constexpr int LA = SplitLds<KA>::bytes;
     constexpr int LB = KB > 0 ? SplitLds<(KB > 0 ? KB : 2)>::bytes : 0;
     __shared__ __attribute__((aligned(16))) char lds[LA > LB ? LA : LB];
@@ -1005,21 +1008,21 @@ split_kernel(SplitParams prm) {
         // which held half the beacon items back until they drained).
         if (w >= prm.seg[0].nwg) {
             split_segment<KB, 1, 0, 0, RAWPG, FQ>(prm.seg[1], w - prm.seg[0].nwg, prm.B, prm.Lq, prm.Hq,
-                                                  prm.scale_log2, lds, nullptr, &prm.rawp, FQ ? &prm.qrope : nullptr,
+                                                  prm.scale_log2, lds, nullptr, &prm.rawp, QR ? &prm.qrope : nullptr,
                                                   nullptr, FQ ? &prm.kshift : nullptr);
             return;
         }
     } else if constexpr (KB > 0) {
         if (w < prm.seg[1].nwg) {
             split_segment<KB, 1, 0, 0, RAWPG, FQ>(prm.seg[1], w, prm.B, prm.Lq, prm.Hq, prm.scale_log2, lds, nullptr,
-                                                  &prm.rawp, FQ ? &prm.qrope : nullptr, nullptr,
+                                                  &prm.rawp, QR ? &prm.qrope : nullptr, nullptr,
                                                   FQ ? &prm.kshift : nullptr);
             return;
         }
         w -= prm.seg[1].nwg;
     }
     split_segment<KA, SplitDepth<KA>::value, PAGED, SEG2, 0, FQ>(prm.seg[0], w, prm.B, prm.Lq, prm.Hq, prm.scale_log2,
-                                                                 lds, &prm.two, nullptr, FQ ? &prm.qrope : nullptr,
+                                                                 lds, &prm.two, nullptr, QR ? &prm.qrope : nullptr,
                                                                  FQ ? &prm.absorb : nullptr);
 }
 
@@ -3397,28 +3400,15 @@ int recon_decode_run(const slimkv_recon_decode_args* r, void* workspace, size_t 
     uint16_t* kbuf = reinterpret_cast<uint16_t*>(ws + p.k_off);
     uint16_t* vbuf = reinterpret_cast<uint16_t*>(ws + p.v_off);
 
-    // 1. query RoPE (no absorption)
-    PrologueParams pp{};
-    pp.q = static_cast<const uint16_t*>(a->q); pp.q_sb = a->q_sb; pp.q_sl = a->q_sl; pp.q_sh = a->q_sh;
-    pp.pos = a->q_positions; pp.pos_sb = a->pos_sb;
-    pp.cos = a->cos; pp.sin = a->sin; pp.rope_rows = a->rope_rows;
-    pp.q_rot = q_rot;
-    pp.wq = 0;
-    pp.B = B; pp.Lq = Lq; pp.Hq = Hq; pp.Hkv = Hkv; pp.D = D; pp.Rk = (int)a->rank_k; pp.parts = 1;
-    pp.scale = (float)a->scale;
-    // The fused reconstruction decode rotates its queries where its split
-    // kernel reads them (no prologue launch; the prologue stage does nothing).
+    // 1. The split kernels rotate the queries where they read them: no prologue
+    // launch (the prologue stage does nothing).
     if (p.fused) return recon_fused_run(r, p, ws, q_rot, st, stages);
-    if (stages & SLIMKV_STAGE_PROLOGUE) {
-        hipLaunchKernelGGL(prologue_kernel, dim3(B * Hkv), dim3(256), 0, st, pp);
-        rc = check_hip(hipGetLastError(), "prologue kernel launch");
-        if (rc != SLIMKV_OK) return rc;
-    }
 
     // 2. rebuild beacon K (optionally RoPE'd) and, unless it stays latent, V: [B, Nl, Hkv, D]
     if (has_lat && (stages & SLIMKV_STAGE_ATTEND)) {
-        for (int kind = 0; kind < (p.v_latent ? 1 : 2); ++kind) {
-            slimkv_reconstruct_args ra{};
+        slimkv_reconstruct_args rebuilt[2] = {};
+        for (int kind = 0; kind < 2; ++kind) {
+            slimkv_reconstruct_args& ra = rebuilt[kind];
             ra.latent = kind ? a->lat_v : a->lat_k;
             ra.l_sb = kind ? a->lv_sb : a->lk_sb;
             ra.l_sn = kind ? a->lv_sn : a->lk_sn;
@@ -3432,9 +3422,9 @@ int recon_decode_run(const slimkv_recon_decode_args* r, void* workspace, size_t 
             }
             ra.batch = B; ra.rows = a->lat_keys; ra.rank = kind ? a->rank_v : a->rank_k;
             ra.kv_heads = Hkv; ra.head_dim = D; ra.block_diagonal = a->block_diagonal;
-            rc = reconstruct(&ra, st);
-            if (rc != SLIMKV_OK) return rc;
         }
+        rc = reconstruct_pair(&rebuilt[0], p.v_latent ? nullptr : &rebuilt[1], st, r->rope_pairs, r->rope_repeats);
+        if (rc != SLIMKV_OK) return rc;
     }
 
     // 3. split-K attention over [rebuilt beacons ; raw rows]
@@ -3442,6 +3432,8 @@ int recon_decode_run(const slimkv_recon_decode_args* r, void* workspace, size_t 
     prm.B = B; prm.Lq = Lq; prm.Hq = Hq;
     prm.scale_log2 = (float)(a->scale * 1.4426950408889634);
     prm.nseg = has_lat ? 2 : 1;
+    prm.qrope = QRope{static_cast<const uint16_t*>(a->q), a->q_sb, a->q_sl, a->q_sh, a->q_positions, a->pos_sb, a->cos,
+                      a->sin, a->rope_rows};
     Seg& rs = prm.seg[has_lat ? 1 : 0];
     rs.q = q_rot; rs.q_sb = (int64_t)Lq * Hq * D; rs.q_sl = (int64_t)Hq * D; rs.q_sh = D;
     rs.k = static_cast<const uint16_t*>(a->raw_k); rs.k_sb = a->rk_sb; rs.k_sn = a->rk_sn; rs.k_sh = a->rk_sh;

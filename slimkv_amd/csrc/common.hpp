@@ -108,6 +108,9 @@ void set_error(const std::string& msg);
 int fail(int code, const std::string& msg);
 int check_hip(hipError_t err, const char* what);
 int device_cu_count();
-int reconstruct(const slimkv_reconstruct_args* a, hipStream_t st);
+// One or two (b non-null) reconstructions; pairs: the rows of a's RoPE tables
+// as slimkv_prepare_rope_pairs makes them, repeats as rope_repeats there.
+int reconstruct_pair(const slimkv_reconstruct_args* a, const slimkv_reconstruct_args* b, hipStream_t st,
+                     const uint32_t* pairs = nullptr, int repeats = 0);
 
 }  // namespace slimkv

@@ -23,6 +23,7 @@ struct ReconParams {
     const int64_t* dst_rows;                                  // [n] or null (identity)
     const float* cos; const float* sin; int64_t rope_rows;
     const int64_t* positions; int64_t pos_sb;                 // [B, n] or null
+    const uint32_t* pairs; int repeats;                       // (bf16 cos | bf16 sin << 16) rows of the tables or null
     int B, n, R, Hkv, blockdiag, k_lo_step;                   // k_lo_step: per-head latent slice width
     int in16, out16;                                          // latent and W / output rows 16-byte aligned
     int tables16;                                             // RoPE tables 16-byte aligned
@@ -331,23 +332,35 @@ __device__ __forceinline__ void recon_wide_body(const ReconParams& p, int segs, 
 #pragma unroll
         for (int i = 0; i < 4; ++i) bias[f][i] = p.bias ? bf16_to_f32(p.bias[(int64_t)h * D + feature(f, 4 * grp + i)]) : 0.f;
 
-    // The RoPE table pieces of a lane's row, loaded before the tile's products.
+    // A lane's (bf16 cos | bf16 sin << 16) pairs, loaded before the tile's
+    // products: from prepared pairs one 16-byte piece serves both operands
+    // where a row repeats its first half, from the fp32 tables four (K rotated
+    // and V of 8192 rows of width 256: 32.6 us as two launches from the
+    // tables, 27.3 as one from the pairs).
     struct RopePiece {
-        float4 c[2], s[2];
+        u32x4 f[2];
     };
     auto load_rope = [&](RopePiece& t, int row) {
         const int64_t pos = clamp_i64(p.positions[(int64_t)b * p.pos_sb + min(row, p.n - 1)], 0, p.rope_rows - 1);
+        if (p.pairs) {
+            const uint32_t* pr = p.pairs + pos * D + 4 * grp;
+            t.f[0] = *reinterpret_cast<const u32x4*>(pr + 16 * wave);
+            t.f[1] = p.repeats ? t.f[0] : *reinterpret_cast<const u32x4*>(pr + 64 + 16 * wave);
+            return;
+        }
 #pragma unroll
         for (int f = 0; f < 2; ++f) {
             const float* cr = p.cos + pos * D + feature(f, 4 * grp);
             const float* sr = p.sin + pos * D + feature(f, 4 * grp);
+            float4 c, s;
             if (p.tables16) {
-                t.c[f] = *reinterpret_cast<const float4*>(cr);
-                t.s[f] = *reinterpret_cast<const float4*>(sr);
+                c = *reinterpret_cast<const float4*>(cr);
+                s = *reinterpret_cast<const float4*>(sr);
             } else {
-                t.c[f] = make_float4(cr[0], cr[1], cr[2], cr[3]);
-                t.s[f] = make_float4(sr[0], sr[1], sr[2], sr[3]);
+                c = make_float4(cr[0], cr[1], cr[2], cr[3]);
+                s = make_float4(sr[0], sr[1], sr[2], sr[3]);
             }
+            t.f[f] = u32x4{pack_bf16(c.x, s.x), pack_bf16(c.y, s.y), pack_bf16(c.z, s.z), pack_bf16(c.w, s.w)};
         }
     };
     auto finish = [&](const v4f (&acc)[2], const RopePiece& t, int row) {
@@ -362,12 +375,11 @@ __device__ __forceinline__ void recon_wide_body(const ReconParams& p, int segs, 
         if constexpr (ROPE) {
 #pragma unroll
             for (int f = 0; f < 2; ++f) {
-                const float cv[4] = {t.c[f].x, t.c[f].y, t.c[f].z, t.c[f].w}, sv[4] = {t.s[f].x, t.s[f].y, t.s[f].z, t.s[f].w};
                 float y[4];
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     const float partner = f == 0 ? -x[1][i] : x[0][i];
-                    y[i] = round_bf16_hw(x[f][i] * round_bf16_hw(cv[i])) + round_bf16_hw(partner * round_bf16_hw(sv[i]));
+                    y[i] = round_bf16_hw(x[f][i] * lo_bf16(t.f[f][i])) + round_bf16_hw(partner * hi_bf16(t.f[f][i]));
                 }
                 *reinterpret_cast<u32x2*>(orow + feature(f, 4 * grp)) = u32x2{pack_bf16(y[0], y[1]), pack_bf16(y[2], y[3])};
             }
@@ -419,11 +431,11 @@ recon_wide_kernel(ReconParams p, int segs) {
 }
 
 // Two reconstructions of one width in one launch, as recon_stream_pair_kernel.
-template <int KS, int RT>
+template <int KS, int RT, bool ROPE>   // ROPE: of the first
 __global__ void __launch_bounds__(kReconWaves * 64) __attribute__((amdgpu_waves_per_eu(2)))
 recon_wide_pair_kernel(ReconParams p0, ReconParams p1, int segs0, int segs1, int blocks0) {
     __shared__ __attribute__((aligned(16))) char lds[WideLds<KS>::bytes];
-    if ((int)blockIdx.x < blocks0) recon_wide_body<KS, RT, false, true>(p0, segs0, blockIdx.x, lds);
+    if ((int)blockIdx.x < blocks0) recon_wide_body<KS, RT, ROPE, true>(p0, segs0, blockIdx.x, lds);
     else recon_wide_body<KS, RT, false, true>(p1, segs1, blockIdx.x - blocks0, lds);
 }
 
@@ -572,33 +584,37 @@ hipError_t launch_wide_pair(const ReconParams& p0, int segs0, const ReconParams&
     const int blocks0 = p0.B * p0.Hkv * segs0;
     const int blocks1 = p1.B * p1.Hkv * segs1;
     const dim3 grid(blocks0 + blocks1), block(kReconWaves * 64);
-    if (p0.row_frags == 1)
-        hipLaunchKernelGGL((recon_wide_pair_kernel<KS, 1>), grid, block, 0, st, p0, p1, segs0, segs1, blocks0);
-    else
-        hipLaunchKernelGGL((recon_wide_pair_kernel<KS, 2>), grid, block, 0, st, p0, p1, segs0, segs1, blocks0);
+#define SLIMKV_PAIR(RT, ROPE) \
+    hipLaunchKernelGGL((recon_wide_pair_kernel<KS, RT, ROPE>), grid, block, 0, st, p0, p1, segs0, segs1, blocks0)
+    if (p0.positions) {
+        if (p0.row_frags == 1) SLIMKV_PAIR(1, true);
+        else SLIMKV_PAIR(2, true);
+    } else {
+        if (p0.row_frags == 1) SLIMKV_PAIR(1, false);
+        else SLIMKV_PAIR(2, false);
+    }
+#undef SLIMKV_PAIR
     return hipGetLastError();
 }
 
-int reconstruct(const slimkv_reconstruct_args* a, hipStream_t st) {
-    ReconParams p;
-    int segs = 0, kw = 0;
-    const int rc = prepare_recon(a, &p, &segs, &kw);
-    if (rc != SLIMKV_OK || a->rows == 0) return rc;
-    return launch_prepared(p, segs, kw, st);
-}
-
-int reconstruct_pair(const slimkv_reconstruct_args* a, const slimkv_reconstruct_args* b, hipStream_t st) {
+int reconstruct_pair(const slimkv_reconstruct_args* a, const slimkv_reconstruct_args* b, hipStream_t st,
+                     const uint32_t* pairs, int repeats) {
     ReconParams pa, pb;
     int sa = 0, sb = 0, ka = 0, kb = 0;
     int rc = prepare_recon(a, &pa, &sa, &ka);
     if (rc != SLIMKV_OK) return rc;
+    if (pairs && pa.positions && pal16(pairs)) {
+        pa.pairs = pairs;
+        pa.repeats = repeats;
+    }
+    if (!b) return a->rows == 0 ? SLIMKV_OK : launch_prepared(pa, sa, ka, st);
     rc = prepare_recon(b, &pb, &sb, &kb);
     if (rc != SLIMKV_OK) return rc;
     if (a->rows == 0) return b->rows == 0 ? SLIMKV_OK : launch_prepared(pb, sb, kb, st);
     if (b->rows == 0) return launch_prepared(pa, sa, ka, st);
-    // wide widths share a launch without RoPE and with 16-byte rows
+    // wide widths share a launch with 16-byte rows and RoPE at most of the first
     const bool pairable =
-        ka <= 64 || (!pa.positions && !pb.positions && pa.in16 && pb.in16 && pa.row_frags == pb.row_frags);
+        ka <= 64 || (!pb.positions && pa.in16 && pb.in16 && pa.row_frags == pb.row_frags);
     if (sa > 0 && sb > 0 && ka == kb && pairable) {
         hipError_t e;
         switch (ka / 16) {
@@ -623,7 +639,7 @@ int reconstruct_pair(const slimkv_reconstruct_args* a, const slimkv_reconstruct_
 }  // namespace slimkv
 
 extern "C" int slimkv_reconstruct(const slimkv_reconstruct_args* a, void* stream) {
-    return slimkv::reconstruct(a, static_cast<hipStream_t>(stream));
+    return slimkv::reconstruct_pair(a, nullptr, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int slimkv_reconstruct_pair(const slimkv_reconstruct_args* a, const slimkv_reconstruct_args* b,

@@ -272,6 +272,22 @@ int slimkv_reconstruct(const slimkv_reconstruct_args* a, void* stream);
  * rebuilt together (a prefill window's beacon rows, modeling_llama.py:1347-1367). */
 int slimkv_reconstruct_pair(const slimkv_reconstruct_args* a, const slimkv_reconstruct_args* b, void* stream);
 
+/* A reconstruction and the full-width rows around it: [sink | up(history) |
+ * raw | current] as ReconstructionCache.materialize concatenates them
+ * (slimkv/llama3/memory.py:26-48).  Copy i moves src[b, h, n, 0..127] (element
+ * strides sb, sh, sn) to row first_row + n of `out`, the same first row of the
+ * output for every copy, with the reconstruction's output strides, batch and
+ * heads; up to three copies, rows 16-byte aligned, not overlapping the output.
+ * One launch at contracted widths of 128 and more, else two. */
+typedef struct slimkv_row_copy {
+    const void* src; int64_t sb, sh, sn;
+    void* out;
+    int64_t first_row, rows;
+} slimkv_row_copy;
+
+int slimkv_reconstruct_with_rows(const slimkv_reconstruct_args* a, const slimkv_row_copy* copies, int32_t count,
+                                 void* stream);
+
 /* ------------------------------------------------------------------------
  * Reconstruction decode for one attention layer: rebuild every beacon's K
  * (RoPE'd at `beacon_positions` when given) and V from the latents, then one

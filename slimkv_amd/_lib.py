@@ -75,6 +75,11 @@ ReconstructArgs = _struct('slimkv_reconstruct_args', [
     ('block_diagonal', c_i32),
 ])
 
+RowCopy = _struct('slimkv_row_copy', [
+    ('src', c_ptr), *_i64s('sb', 'sh', 'sn'),
+    ('out', c_ptr), *_i64s('first_row', 'rows'),
+])
+
 ReconDecodeArgs = _struct('slimkv_recon_decode_args', [
     ('base', LatentDecodeArgs),
     ('beacon_positions', c_ptr), ('bpos_sb', c_i64),
@@ -244,6 +249,8 @@ SIGNATURES = {
     'slimkv_prepare_rope_pairs': (ctypes.c_int, [c_ptr, c_ptr, c_i64, c_i64, c_ptr, c_ptr]),
     'slimkv_reconstruct': (ctypes.c_int, [ctypes.POINTER(ReconstructArgs), c_ptr]),
     'slimkv_reconstruct_pair': (ctypes.c_int, [ctypes.POINTER(ReconstructArgs), ctypes.POINTER(ReconstructArgs), c_ptr]),
+    'slimkv_reconstruct_with_rows': (ctypes.c_int, [ctypes.POINTER(ReconstructArgs), ctypes.POINTER(RowCopy), c_i32,
+                                                    c_ptr]),
     'slimkv_recon_decode_workspace': (ctypes.c_size_t, [ctypes.POINTER(ReconDecodeArgs)]),
     'slimkv_recon_decode': (ctypes.c_int, [ctypes.POINTER(ReconDecodeArgs), c_ptr, ctypes.c_size_t, c_ptr]),
     'slimkv_recon_decode_stages': (ctypes.c_int, [ctypes.POINTER(ReconDecodeArgs), ctypes.c_int, c_ptr,

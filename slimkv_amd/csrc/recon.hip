@@ -439,6 +439,67 @@ recon_wide_pair_kernel(ReconParams p0, ReconParams p1, int segs0, int segs1, int
     else recon_wide_body<KS, RT, false, true>(p1, segs1, blockIdx.x - blocks0, lds);
 }
 
+// Full-width rows beside the rebuilt ones ([sink | history | raw | current] of
+// a history rebuild): copied by extra workgroups of the same launch, 64 rows
+// each, sixteen lanes a 256-byte row.
+struct RowCopies {
+    static constexpr int kMax = 3;
+    const uint16_t* src[kMax]; int64_t sb[kMax], sh[kMax], sn[kMax];
+    int64_t dst_row[kMax];                                    // first row of the output
+    int rows[kMax], groups[kMax];                             // rows of a head, workgroups (0: no such copy)
+    int count;
+};
+constexpr int kCopyRows = 64;
+
+__device__ __forceinline__ void copy_rows(const RowCopies& c, const ReconParams& p, int block) {
+    // One call per copy: an index into the kernel arguments, or a select
+    // between their fields, would put them in scratch memory.
+    auto copy = [&](const uint16_t* src, int64_t sb, int64_t sh, int64_t sn, int64_t dst_row, int rows, int at_block) {
+        const int total = p.B * p.Hkv * rows;
+        const int piece = 8 * (threadIdx.x & 15);
+        u32x4 v[kCopyRows / 16];
+        int64_t at[kCopyRows / 16];
+#pragma unroll
+        for (int u = 0; u < kCopyRows / 16; ++u) {
+            // past the end: the last row again
+            const int r = min(at_block * kCopyRows + 16 * u + (int)(threadIdx.x >> 4), total - 1);
+            const int n = r % rows, h = r / rows % p.Hkv, b = r / rows / p.Hkv;
+            v[u] = *reinterpret_cast<const u32x4*>(src + b * sb + h * sh + n * sn + piece);
+            at[u] = b * p.o_sb + h * p.o_sh + (dst_row + n) * p.o_sn + piece;
+        }
+#pragma unroll
+        for (int u = 0; u < kCopyRows / 16; ++u) *reinterpret_cast<u32x4*>(p.out + at[u]) = v[u];
+    };
+    if (block < c.groups[0]) {
+        copy(c.src[0], c.sb[0], c.sh[0], c.sn[0], c.dst_row[0], c.rows[0], block);
+        return;
+    }
+    block -= c.groups[0];
+    if (block < c.groups[1]) {
+        copy(c.src[1], c.sb[1], c.sh[1], c.sn[1], c.dst_row[1], c.rows[1], block);
+        return;
+    }
+    copy(c.src[2], c.sb[2], c.sh[2], c.sn[2], c.dst_row[2], c.rows[2], block - c.groups[1]);
+}
+
+__global__ void __launch_bounds__(kReconWaves * 64) copy_rows_kernel(ReconParams p, RowCopies c) {
+    copy_rows(c, p, blockIdx.x);
+}
+
+// `shift`: the copies' rows count from the output's first row, the rebuilt ones
+// from p.out + shift.
+template <int KS, int RT>
+__global__ void __launch_bounds__(kReconWaves * 64) __attribute__((amdgpu_waves_per_eu(2)))
+recon_wide_copies_kernel(ReconParams p, int segs, int blocks, int64_t shift, RowCopies c) {
+    __shared__ __attribute__((aligned(16))) char lds[WideLds<KS>::bytes];
+    if ((int)blockIdx.x >= blocks) {
+        copy_rows(c, p, blockIdx.x - blocks);
+        return;
+    }
+    p.out += shift;
+    recon_wide_body<KS, RT, false, true>(p, segs, blockIdx.x, lds);
+}
+
 namespace {
 bool al4(int64_t x) { return (x & 3) == 0; }
 bool pal8(const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 7) == 0; }
@@ -636,7 +697,82 @@ int reconstruct_pair(const slimkv_reconstruct_args* a, const slimkv_reconstruct_
     return rc != SLIMKV_OK ? rc : launch_prepared(pb, sb, kb, st);
 }
 
+namespace {
+
+template <int KS>
+hipError_t launch_wide_copies(const ReconParams& p, int segs, int64_t shift, const RowCopies& c, int groups,
+                              hipStream_t st) {
+    const int blocks = p.B * p.Hkv * segs;
+    const dim3 grid(blocks + groups), block(kReconWaves * 64);
+    if (p.row_frags == 1)
+        hipLaunchKernelGGL((recon_wide_copies_kernel<KS, 1>), grid, block, 0, st, p, segs, blocks, shift, c);
+    else
+        hipLaunchKernelGGL((recon_wide_copies_kernel<KS, 2>), grid, block, 0, st, p, segs, blocks, shift, c);
+    return hipGetLastError();
+}
+
+}  // namespace
+
+int reconstruct_with_rows(const slimkv_reconstruct_args* a, const slimkv_row_copy* copies, int count, hipStream_t st) {
+    if (!a || count < 0 || count > RowCopies::kMax || (count && !copies)) return fail(SLIMKV_EINVAL, "invalid row copies");
+    ReconParams p{};
+    int segs = 0, kw = 0;
+    int rc = prepare_recon(a, &p, &segs, &kw);
+    if (rc != SLIMKV_OK) return rc;
+    RowCopies c{};
+    void* out = nullptr;
+    int64_t groups = 0;
+    for (int i = 0; i < count; ++i) {
+        const slimkv_row_copy& r = copies[i];
+        if (r.rows < 0 || r.first_row < 0 || a->batch * a->kv_heads * r.rows > (1 << 30))
+            return fail(SLIMKV_EINVAL, "invalid row copy");
+        if (r.rows == 0) continue;
+        if (!r.src || !r.out || !pal16(r.src) || !pal16(r.out) || !al8(r.sb) || !al8(r.sn) || !al8(r.sh) ||
+            !al8(a->o_sb) || !al8(a->o_sn) || !al8(a->o_sh))
+            return fail(SLIMKV_EINVAL, "row copies need 16-byte aligned rows");
+        if (c.count && r.out != out) return fail(SLIMKV_EINVAL, "row copies share one output");
+        out = r.out;
+        c.src[c.count] = static_cast<const uint16_t*>(r.src);
+        c.sb[c.count] = r.sb; c.sh[c.count] = r.sh; c.sn[c.count] = r.sn;
+        c.dst_row[c.count] = r.first_row;
+        c.rows[c.count] = (int)r.rows;
+        c.groups[c.count] = (int)((a->batch * a->kv_heads * r.rows + kCopyRows - 1) / kCopyRows);
+        groups += c.groups[c.count++];
+    }
+    if (!c.count) return a->rows == 0 ? SLIMKV_OK : launch_prepared(p, segs, kw, st);
+    ReconParams whole = p;
+    if (a->rows == 0) {
+        whole.B = (int)a->batch; whole.Hkv = (int)a->kv_heads;
+        whole.o_sb = a->o_sb; whole.o_sn = a->o_sn; whole.o_sh = a->o_sh;
+    }
+    whole.out = static_cast<uint16_t*>(out);
+    if (a->rows > 0 && kw >= 128 && !p.positions && p.in16 && p.out16) {
+        const int64_t shift = p.out - whole.out;
+        hipError_t e;
+        switch (kw / 16) {
+            case 8: e = launch_wide_copies<4>(whole, segs, shift, c, (int)groups, st); break;
+            case 12: e = launch_wide_copies<6>(whole, segs, shift, c, (int)groups, st); break;
+            case 16: e = launch_wide_copies<8>(whole, segs, shift, c, (int)groups, st); break;
+            case 24: e = launch_wide_copies<12>(whole, segs, shift, c, (int)groups, st); break;
+            case 32: e = launch_wide_copies<16>(whole, segs, shift, c, (int)groups, st); break;
+            default: return fail(SLIMKV_EUNSUP, "latent width not instantiated");
+        }
+        return check_hip(e, "reconstruction kernel launch");
+    }
+    if (a->rows > 0) {
+        rc = launch_prepared(p, segs, kw, st);
+        if (rc != SLIMKV_OK) return rc;
+    }
+    hipLaunchKernelGGL(copy_rows_kernel, dim3((unsigned)groups), dim3(kReconWaves * 64), 0, st, whole, c);
+    return check_hip(hipGetLastError(), "row copy launch");
+}
+
 }  // namespace slimkv
+
+extern "C" int slimkv_reconstruct_with_rows(const slimkv_reconstruct_args* a, const slimkv_row_copy* copies,
+                                            int32_t count, void* stream) {
+    return slimkv::reconstruct_with_rows(a, copies, count, static_cast<hipStream_t>(stream));
+}
 
 extern "C" int slimkv_reconstruct(const slimkv_reconstruct_args* a, void* stream) {
     return slimkv::reconstruct_pair(a, nullptr, static_cast<hipStream_t>(stream));

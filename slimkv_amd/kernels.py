@@ -500,6 +500,30 @@ def reconstruct_pair(first, second):
     return out_a, out_b
 
 
+def reconstruct_with_rows(latent, weight, bias, out, first_row, parts, *, block_diagonal=False):
+    """Up-projected latent rows [B, n, R] at rows first_row .. first_row + n - 1
+    of out [B, Hkv, total, D] and full-width rows beside them: parts, up to
+    three (row, tensor [B, Hkv, m, D]) pairs, each copied to rows row .. row +
+    m - 1.  One launch where the library can (contracted widths of 128 and
+    more).  Returns out."""
+    _need_device(*(t for _, t in parts))
+    _need_bf16(*(t for _, t in parts))
+    heads, n = out.shape[1], latent.shape[1]
+    a, _, keep = _reconstruct_args(latent, weight, bias, heads, out[:, :, first_row:first_row + n].transpose(1, 2), None,
+                                   None, None, None, block_diagonal)
+    copies = (_lib.RowCopy * len(parts))()
+    base = out.data_ptr()
+    for c, (row, t) in zip(copies, parts):
+        if t.dim() != 4 or t.shape[:2] != out.shape[:2] or t.shape[3] != out.shape[3] or t.stride(3) != 1 or \
+                row < 0 or row + t.shape[2] > out.shape[2]:
+            raise ValueError('parts must be [B, Hkv, m, D] rows inside the output')
+        c.src, c.out, c.first_row, c.rows = t.data_ptr(), base, row, t.shape[2]
+        c.sb, c.sh, c.sn = t.stride()[:3]
+    check(lib().slimkv_reconstruct_with_rows(ctypes.byref(a), copies, len(parts), _lib.stream_handle(out.device)))
+    del keep
+    return out
+
+
 def _recon_kwargs(kw):
     names = ('latent', 'weight', 'bias', 'kv_heads', 'out', 'dst_rows', 'positions', 'cos', 'sin', 'block_diagonal')
     unknown = set(kw) - set(names)

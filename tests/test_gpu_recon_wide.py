@@ -64,3 +64,36 @@ def test_wide_pair_equals_single_launches(device, rows):
     problems = [dict(zip(('latent', 'weight', 'bias'), _inputs(device, 1, n, 256, 0)), kv_heads=HKV) for n in rows]
     for got, kw in zip(kernels.reconstruct_pair(*problems), problems):
         assert torch.equal(got, kernels.reconstruct(**kw))
+
+
+@pytest.mark.parametrize('rank,per_head,B,sink,n,raw,current', [(256, False, 2, 4, 300, 0, 70), (128, False, 1, 1, 17, 33, 1),
+                                                                (512, False, 1, 0, 16, 5, 64), (32, True, 3, 4, 65, 7, 0),
+                                                                (384, False, 2, 0, 1, 0, 129)])
+def test_rows_around_a_rebuilt_history(device, rank, per_head, B, sink, n, raw, current):
+    """[sink | up(history) | raw | current] in one call: the rebuilt rows are
+    reconstruct's bits, the others copies, from strided and offset parts."""
+    from types import SimpleNamespace
+    from slimkv_amd import kernels
+    from slimkv_amd.memory import ReconstructionCache
+    from slimkv_amd.workloads import block_diagonal
+    gen = torch.Generator(device=device).manual_seed(rank + n)
+
+    def rnd(*shape):
+        return torch.randn(*shape, generator=gen, device=device).to(torch.bfloat16)
+    R = HKV * rank if per_head else rank
+    up = torch.nn.Linear(R, HKV * D, bias=True, device=device, dtype=torch.bfloat16).requires_grad_(False)
+    if per_head:
+        up.weight.copy_(block_diagonal([rnd(D, rank) for _ in range(HKV)]))
+    parts = [rnd(B, HKV, sink + 3, D)[:, :, 3:] if sink else None, rnd(B, raw, HKV, D).transpose(1, 2) if raw else None,
+             rnd(B, current, HKV, 2 * D)[..., D:].transpose(1, 2) if current else None]
+    latent = rnd(B, 1, n, R)
+    cache = ReconstructionCache(parts[0], latent, parts[1], None, None, HKV, D, 'k')
+    attention = SimpleNamespace(beacon_k_up_proj=up, num_key_value_heads=HKV, head_dim=D)
+    got = cache.materialize(attention, parts[2])
+    rebuilt = kernels.reconstruct(latent[:, 0], up.weight, up.bias, kv_heads=HKV, block_diagonal=per_head)
+    want = torch.cat([x for x in (parts[0], rebuilt.transpose(1, 2), parts[1], parts[2]) if x is not None], 2)
+    assert torch.equal(got, want)
+    if current:                     # rows off a 16-byte boundary are copied by torch: the same result
+        shifted = torch.empty(parts[2].numel() + 1, dtype=torch.bfloat16, device=device)[1:].view(parts[2].shape)
+        shifted.copy_(parts[2])
+        assert torch.equal(cache.materialize(attention, shifted), want)

@@ -1492,6 +1492,34 @@ __device__ __forceinline__ int live_b_splits(const CombineParams& cp, int b) {
     return min(cp.b_splits, (len + cp.b_rps - 1) / cp.b_rps);
 }
 
+template <int CTRL>
+__device__ __forceinline__ float dpp_f(float v) {
+    return __uint_as_float(__builtin_amdgcn_mov_dpp(__float_as_uint(v), CTRL, 0xf, 0xf, true));
+}
+// Over all 64 lanes: row_ror 1, 2, 4, 8 inside each 16-lane row, then the
+// row swaps.  Each lane's sum associates in its own rotation order, so lanes
+// may hold sums an fp32 ulp apart (deterministic for given inputs); callers
+// that need one value on every lane take lane 0's (wave_first).
+__device__ __forceinline__ float wave_max64(float v) {
+    v = fmaxf(v, dpp_f<0x121>(v));
+    v = fmaxf(v, dpp_f<0x122>(v));
+    v = fmaxf(v, dpp_f<0x124>(v));
+    v = fmaxf(v, dpp_f<0x128>(v));
+    return rows_max(v);
+}
+__device__ __forceinline__ float wave_sum64(float v) {
+    v += dpp_f<0x121>(v);
+    v += dpp_f<0x122>(v);
+    v += dpp_f<0x124>(v);
+    v += dpp_f<0x128>(v);
+    return rows_sum(v);
+}
+
+// Lane 0's value on every lane (a scalar register).
+__device__ __forceinline__ float wave_first(float v) {
+    return __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(v)));
+}
+
 // One workgroup per (b, query head, query): LSE-merge the split partials of
 // both segments, lift the latent accumulator through U_V, fold the biases --
 // for every shape the two narrower kernels below do not take (latents of all
@@ -1574,30 +1602,23 @@ combine_kernel(CombineParams cp) {
         lv = bml[2 * (t - cp.a_splits) + 1];
         if (mv != kNegInf) mv += shift;
     }
-    auto wave_reduce = [](float v, auto op) {
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) v = op(v, shfl_xor_f(v, o));
-        return v;
-    };
-    auto maxf = [](float x, float y) { return fmaxf(x, y); };
-    auto addf = [](float x, float y) { return x + y; };
     const int lane = t & 63, wave = t >> 6;
-    const float wm = wave_reduce(mv, maxf);
+    const float wm = wave_max64(mv);
     if (lane == 0) red[0][wave] = wm;
     __syncthreads();
-    const float M = wave_reduce(lane < NW ? red[0][lane] : kNegInf, maxf);
+    const float M = wave_max64(lane < NW ? red[0][lane] : kNegInf);
     const float Mref = M == kNegInf ? 0.f : M;
     const float wgt = mv == kNegInf ? 0.f : fast_exp2(mv - Mref);
     if (t < total) wts[t] = wgt;
-    const float la = wave_reduce(t < cp.a_splits ? lv * wgt : 0.f, addf);
-    const float lb = wave_reduce(t >= cp.a_splits ? lv * wgt : 0.f, addf);
+    const float la = wave_sum64(t < cp.a_splits ? lv * wgt : 0.f);
+    const float lb = wave_sum64(t >= cp.a_splits ? lv * wgt : 0.f);
     if (lane == 0) {
         red[1][wave] = la;
         red[2][wave] = lb;
     }
     __syncthreads();
-    const float LA = wave_reduce(lane < NW ? red[1][lane] : 0.f, addf);
-    const float LB = wave_reduce(lane < NW ? red[2][lane] : 0.f, addf);
+    const float LA = wave_first(wave_sum64(lane < NW ? red[1][lane] : 0.f));
+    const float LB = wave_first(wave_sum64(lane < NW ? red[2][lane] : 0.f));
     const float L = LA + LB;
 
     // Weighted quad sums of the thread's splits, then over the split groups.
@@ -1653,8 +1674,10 @@ combine_kernel(CombineParams cp) {
                     sum += lo_bf16(w[i].w) * x1.z + hi_bf16(w[i].w) * x1.w;
                 }
             }
-#pragma unroll
-            for (int o = 4; o > 0; o >>= 1) sum += shfl_xor_f(sum, o);
+            // over the eight lanes: quad permutes, then the half row mirrored
+            sum += dpp_f<0xb1>(sum);
+            sum += dpp_f<0x4e>(sum);
+            sum += dpp_f<0x141>(sum);
             if (piece == 0) {
                 sum += acca[d];
                 if (cp.up_v_bias) sum += bf16_to_f32(cp.up_v_bias[(int64_t)h * cp.D + d]) * LB;
@@ -1779,9 +1802,7 @@ combine_fast_kernel(CombineParams cp) {
     // slots in red[], so no barrier guards their reuse).
     constexpr int NW = T / 64;
     const int wave = t >> 6;
-    float M = mv;
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) M = fmaxf(M, shfl_xor_f(M, o));
+    float M = wave_max64(mv);
     if ((t & 63) == 0) red[wave] = M;
     __syncthreads();
     M = red[0];
@@ -1790,13 +1811,8 @@ combine_fast_kernel(CombineParams cp) {
     const float Mref = M == kNegInf ? 0.f : M;
     const float wgt = (t < total && mv != kNegInf) ? fast_exp2(mv - Mref) : 0.f;
     if (t < total) wts[t] = wgt;
-    float LA = t < cp.a_splits ? lv * wgt : 0.f;
-    float LB = t >= cp.a_splits && t < total ? lv * wgt : 0.f;
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        LA += shfl_xor_f(LA, o);
-        LB += shfl_xor_f(LB, o);
-    }
+    float LA = wave_sum64(t < cp.a_splits ? lv * wgt : 0.f);
+    float LB = wave_sum64(t >= cp.a_splits && t < total ? lv * wgt : 0.f);
     if ((t & 63) == 0) {
         red[NW + 2 * wave] = LA;
         red[NW + 2 * wave + 1] = LB;
@@ -1890,34 +1906,6 @@ bool combine_fast_ok(const CombineParams& cp, int T) {
 // wave's own LDS; a lane owns output columns 2 * lane and 2 * lane + 1.
 constexpr int kWaveRaw = 8;         // raw splits
 constexpr int kWaveLat = 4;         // latent partial quads per lane
-
-template <int CTRL>
-__device__ __forceinline__ float dpp_f(float v) {
-    return __uint_as_float(__builtin_amdgcn_mov_dpp(__float_as_uint(v), CTRL, 0xf, 0xf, true));
-}
-// Over all 64 lanes: row_ror 1, 2, 4, 8 inside each 16-lane row, then the
-// row swaps.  Each lane's sum associates in its own rotation order, so lanes
-// may hold sums an fp32 ulp apart (deterministic for given inputs); callers
-// that need one value on every lane take lane 0's (wave_first).
-__device__ __forceinline__ float wave_max64(float v) {
-    v = fmaxf(v, dpp_f<0x121>(v));
-    v = fmaxf(v, dpp_f<0x122>(v));
-    v = fmaxf(v, dpp_f<0x124>(v));
-    v = fmaxf(v, dpp_f<0x128>(v));
-    return rows_max(v);
-}
-__device__ __forceinline__ float wave_sum64(float v) {
-    v += dpp_f<0x121>(v);
-    v += dpp_f<0x122>(v);
-    v += dpp_f<0x124>(v);
-    v += dpp_f<0x128>(v);
-    return rows_sum(v);
-}
-
-// Lane 0's value on every lane (a scalar register).
-__device__ __forceinline__ float wave_first(float v) {
-    return __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(v)));
-}
 
 template <int LW>   // latent width bound (own block), a multiple of 8
 __global__ void __launch_bounds__(64)

@@ -363,5 +363,10 @@ def check(code):
 
 
 def stream_handle(device):
+    """Address of torch's current stream on `device` (a torch.device or what
+    torch.device takes), without building a Stream object for it."""
     import torch
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    if not isinstance(device, torch.device):
+        device = torch.device(device)
+    index = torch.cuda.current_device() if device.index is None else device.index
+    return torch._C._cuda_getCurrentRawStream(index)

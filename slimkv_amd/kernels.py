@@ -17,23 +17,28 @@ BF16 = torch.bfloat16
 
 
 def _ptr(t):
-    return ctypes.c_void_p(0 if t is None else t.data_ptr())
+    # an address (or None): ctypes converts it where it is stored or passed
+    return None if t is None else t.data_ptr()
 
 
 def _need_device(*tensors):
     for t in tensors:
-        if t is not None and t.device.type != 'cuda':
+        if t is not None and not t.is_cuda:
             raise ValueError('slimkv_amd kernels need device tensors (no CPU path)')
 
 
 def _need_bf16(*tensors):
     for t in tensors:
-        if t is not None and t.dtype != BF16:
+        if t is not None and t.dtype is not BF16:
             raise ValueError(f'expected bfloat16, found {t.dtype}')
 
 
 def _last_contiguous(t):
     return t if t.stride(-1) == 1 else t.contiguous()
+
+
+def _int64(t):
+    return t if t.dtype is torch.int64 else t.to(torch.int64)
 
 
 def _workspace(nbytes, device):
@@ -108,7 +113,7 @@ def prefill_attention(q, k, v, scale, causal=True, seqlens_k=None, out=None, lse
         if cos.dim() != 2 or cos.shape[1] != D:
             raise ValueError('RoPE tables must be fp32 [rows, head_dim]')
         pairs, repeats = prepare_rope_pairs(cos, sin)
-        q_positions = q_positions.to(torch.int64)
+        q_positions = _int64(q_positions)
         if q_positions.stride(-1) != 1:
             q_positions = q_positions.contiguous()
         if q_positions.dim() != 2 or q_positions.shape[0] != B or q_positions.shape[1] < Lq:
@@ -174,7 +179,7 @@ def _down_args(x, weight, rows, blocks, out):
     B, L, K = x.shape
     N = weight.shape[0]
     if rows is not None:
-        rows = rows.to(dtype=torch.long).contiguous()
+        rows = _int64(rows).contiguous()
     n = L if rows is None else rows.numel()
     if out is None:
         out = torch.empty(B, n, N, dtype=BF16, device=x.device)
@@ -211,7 +216,7 @@ def down_project_to_pages(x, weight, pages, table, layout, start, kind, rows=Non
     table = table if table.stride(1) == 1 else table.contiguous()
     B, L, K = x.shape
     if rows is not None:
-        rows = rows.to(dtype=torch.long).contiguous()
+        rows = _int64(rows).contiguous()
     n = L if rows is None else rows.numel()
     a = _lib.DownProjectArgs(_ptr(x), x.stride(0), x.stride(1), _ptr(rows), n, L, _ptr(weight),
                              _ptr(pages), 0, 0, B, K, N, int(blocks))
@@ -300,7 +305,7 @@ def _latent_args(q, raw_k, raw_v, lat_k, lat_v, up_k, up_v, scale, up_k_bias, up
             if cos.shape[0] < B * Lq or sin.shape != cos.shape:
                 raise ValueError('RoPE rows at the query positions must cover [B, Lq, D]')
         else:
-            q_positions = q_positions.to(torch.int64)
+            q_positions = _int64(q_positions)
             if q_positions.stride(-1) != 1:
                 q_positions = q_positions.contiguous()
         cos, sin = cos.contiguous(), sin.contiguous()
@@ -547,7 +552,7 @@ def _reconstruct_args(latent, weight, bias, kv_heads, out, dst_rows, positions, 
     if dst_rows is not None:
         dst_rows = dst_rows.to(device=latent.device, dtype=torch.int64).contiguous()
     if positions is not None:
-        positions = positions.to(torch.int64)
+        positions = _int64(positions)
         positions = positions if positions.stride(-1) == 1 else positions.contiguous()
     a = _lib.ReconstructArgs(
         _ptr(latent), latent.stride(0), latent.stride(1), _ptr(weight), _ptr(bias),
@@ -573,7 +578,7 @@ def recon_decode(q, raw_k, raw_v, lat_k, lat_v, up_k, up_v, scale, *, beacon_pos
                                         lat_lengths, raw_splits, lat_splits, out, lse, prepared_bases=False)
     pairs = None
     if beacon_positions is not None:
-        beacon_positions = beacon_positions.to(torch.int64)
+        beacon_positions = _int64(beacon_positions)
         beacon_positions = beacon_positions if beacon_positions.stride(-1) == 1 else beacon_positions.contiguous()
         if cos is None:
             raise ValueError('beacon RoPE needs the cos/sin tables')
@@ -715,8 +720,7 @@ def decode_qkv(x, weight, bias, heads, kv_heads, cos, sin, positions, raw_k, raw
     if status is None and torch.cuda.is_current_stream_capturing():
         raise ValueError('decode_qkv under graph capture needs a caller status word')
     status, owned = _status_word(status, x.device)
-    pos = positions.to(torch.int64)
-    slot = slot_index.to(torch.int64)
+    pos, slot = _int64(positions), _int64(slot_index)
     a = _lib.DecodeQKVArgs(_ptr(x), x.stride(0), _ptr(weight), _ptr(bias), _ptr(q_out), q_out.stride(0),
                            _ptr(raw_k), _ptr(plain_k), _ptr(raw_v), raw_k.stride(0), raw_k.stride(1), _ptr(slot),
                            _ptr(cos), _ptr(sin), cos.shape[0], _ptr(pos), pos.stride(0) if pos.dim() else 1,
@@ -955,7 +959,7 @@ def paged_step_rows(raw_pages, raw_table, beacon_pages, beacon_table, new_k, new
     if cos.dtype != torch.float32 or sin.shape != cos.shape or cos.dim() != 2 or cos.shape[1] != D:
         raise ValueError('RoPE tables must be fp32 [rows, head_dim]')
     cos, sin = cos.contiguous(), sin.contiguous()
-    positions = positions.to(torch.int64)
+    positions = _int64(positions)
     positions = positions if positions.stride(-1) == 1 else positions.contiguous()
     if positions.shape[0] != B or positions.shape[1] < rows:
         raise ValueError('positions must be [B, >= rows]')

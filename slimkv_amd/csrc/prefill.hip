@@ -43,10 +43,10 @@ namespace {
 constexpr int kD = 128;                  // head dim
 constexpr int kQRows = 128;              // query rows per workgroup
 constexpr int kKeys = 64;                // keys per tile
-// Row paddings of 16 elements: 2 % faster than 8 (fewer LDS bank-conflict
-// cycles), and two workgroups' buffers (2 x 77,824 B) still fit a CU's LDS.
+// K rows padded by 16 elements: 2 % faster than 8 (fewer LDS bank-conflict
+// cycles), and two workgroups' buffers (2 x 73,728 B) still fit a CU's LDS.
 constexpr int kKStride = kD + 16;        // K tile row (bf16), 288 B
-constexpr int kVStride = kKeys + 16;     // V^T tile row (bf16), 160 B: 16-byte aligned reads
+constexpr int kVStride = kKeys + 8;      // V^T tile row (bf16), 144 B: 16-byte aligned reads
 constexpr int kXcds = 8;
 
 struct PrefillParams {
@@ -115,8 +115,14 @@ __device__ __forceinline__ void rope_q_operand(u32x4 (&x)[4], const QPairs& t) {
 // side: key 16h + 4g + j of the step sits at 8g + 4h + j, so the eight keys of
 // lane group g (4g + j and 16 + 4g + j, the P^T contraction order) are one
 // 16-byte read.
-__device__ __forceinline__ int vt_pos(int kq) {       // kq: group of 4 keys in the 64-key tile
-    return 32 * (kq >> 3) + 8 * (kq & 3) + 4 * ((kq >> 2) & 1);
+//
+// The 16-byte chunks of a V^T row are XORed with bits 3-5 of its d: the lanes
+// that load one key row in order (whole cache lines; with sixteen rows per
+// sixteen lanes the 32K-token window took 284 us instead of 281) hold d-pieces
+// 8 rows apart (8 x 144 B, two bank groups), and the XOR spreads their 8-byte
+// writes over eight groups.  The eight rows of one operand read share the XOR.
+__device__ __forceinline__ int vt_pos(int kq, int cp) {   // kq: group of 4 keys in the tile, cp: d-piece of 8
+    return 8 * ((4 * (kq >> 3) + (kq & 3)) ^ (cp & 7)) + 4 * ((kq >> 2) & 1);
 }
 
 // bf16 element e of a and of b side by side: (a_e | b_e << 16), one byte
@@ -146,7 +152,7 @@ __device__ __forceinline__ TileOffsets tile_offsets(int64_t k_sn, int64_t v_sn) 
         const int p = tid + 256 * r;
         o.k[r] = (uint32_t)(2 * ((p >> 4) * k_sn + 8 * (p & 15)));
     }
-    const int kq = tid & 15, cp = tid >> 4;
+    const int kq = tid >> 4, cp = tid & 15;
 #pragma unroll
     for (int r = 0; r < 4; ++r) o.v[r] = (uint32_t)(2 * ((4 * kq + r) * v_sn + 8 * cp));   // keys 4kq + r, d-piece cp
     return o;
@@ -177,13 +183,13 @@ __device__ __forceinline__ void store_tile(const TileRegs& t, uint16_t* ks, uint
         const int p = tid + 256 * r;
         *reinterpret_cast<u32x4*>(ks + (p >> 4) * kKStride + 8 * (p & 15)) = t.k[r];
     }
-    const int kq = tid & 15, cp = tid >> 4;
+    const int kq = tid >> 4, cp = tid & 15;
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
         u32x2 w;
         w.x = pair_of(t.v[0], t.v[1], e);
         w.y = pair_of(t.v[2], t.v[3], e);
-        *reinterpret_cast<u32x2*>(vts + (8 * cp + e) * kVStride + vt_pos(kq)) = w;
+        *reinterpret_cast<u32x2*>(vts + (8 * cp + e) * kVStride + vt_pos(kq, cp)) = w;
     }
 }
 
@@ -273,6 +279,10 @@ prefill_kernel(PrefillParams p) {
         if (ntiles > 1) load_tile(tr, kb, vb, p.k_sn, p.v_sn, kKeys, n, toff);
     }
     if (ntiles > 0) __syncthreads();
+    // V^T operand offsets: chunk c of row 16 md + col sits at c ^ (2 md + col / 8) % 8
+    int vrow[4];
+#pragma unroll
+    for (int x = 0; x < 4; ++x) vrow[x] = col * kVStride + 8 * ((2 * x) ^ grp ^ (col >> 3));
     // the wave's earliest query sees keys up to q0 + shift
     const int wave_last = p.causal ? q0 + shift : n - 1;
 
@@ -350,7 +360,8 @@ prefill_kernel(PrefillParams p) {
         for (int ss = 0; ss < 2; ++ss) {
 #pragma unroll
             for (int md = 0; md < 8; ++md) {
-                const u32x4 a = *reinterpret_cast<const u32x4*>(vts + (16 * md + col) * kVStride + 32 * ss + 8 * grp);
+                // row 16 md + col, chunk 4 ss + grp of it
+                const u32x4 a = *reinterpret_cast<const u32x4*>(vts + 16 * md * kVStride + vrow[(2 * ss) ^ (md & 3)]);
 #pragma unroll
                 for (int nt = 0; nt < 2; ++nt) o[md][nt] = mfma32(a, pb[ss][nt], o[md][nt]);
             }

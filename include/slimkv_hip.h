@@ -534,6 +534,14 @@ typedef struct slimkv_prefill_attention_args {
 
 int slimkv_prefill_attention(const slimkv_prefill_attention_args* a, void* stream);
 
+/* The same call with a workspace of slimkv_prefill_attention_workspace(a)
+ * bytes (16-byte aligned; 0: none is used): few long query blocks are then
+ * split over their keys so that every CU ends at the same time, and merged in
+ * fp32.  With a smaller workspace the call runs unsplit. */
+size_t slimkv_prefill_attention_workspace(const slimkv_prefill_attention_args* a);
+int slimkv_prefill_attention_split(const slimkv_prefill_attention_args* a, void* workspace, size_t workspace_bytes,
+                                   void* stream);
+
 /* ------------------------------------------------------------------------
  * Beacon down-projection of the selected rows of a window.
  * Replaces beacon_{k,v}_down_proj inside _project_beacon_key/_value and the

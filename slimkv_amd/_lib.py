@@ -263,6 +263,9 @@ SIGNATURES = {
     'slimkv_merge_typed': (ctypes.c_int, [ctypes.POINTER(MergeArgs), ctypes.c_int, c_ptr]),
     'slimkv_eager_attention': (ctypes.c_int, [ctypes.POINTER(EagerAttentionArgs), c_ptr]),
     'slimkv_prefill_attention': (ctypes.c_int, [ctypes.POINTER(PrefillAttentionArgs), c_ptr]),
+    'slimkv_prefill_attention_workspace': (ctypes.c_size_t, [ctypes.POINTER(PrefillAttentionArgs)]),
+    'slimkv_prefill_attention_split': (ctypes.c_int, [ctypes.POINTER(PrefillAttentionArgs), c_ptr, ctypes.c_size_t,
+                                                      c_ptr]),
     'slimkv_down_project_workspace': (ctypes.c_size_t, [ctypes.POINTER(DownProjectArgs)]),
     'slimkv_down_project': (ctypes.c_int, [ctypes.POINTER(DownProjectArgs), c_ptr, ctypes.c_size_t, c_ptr]),
     'slimkv_down_project_pair_workspace': (ctypes.c_size_t, [ctypes.POINTER(DownProjectArgs),

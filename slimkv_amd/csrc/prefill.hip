@@ -36,6 +36,8 @@
 
 #include "common.hpp"
 
+#include <algorithm>
+
 namespace slimkv {
 
 namespace {
@@ -193,32 +195,43 @@ __device__ __forceinline__ void store_tile(const TileRegs& t, uint16_t* ks, uint
     }
 }
 
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
-prefill_kernel(PrefillParams p) {
-    __shared__ __attribute__((aligned(16))) uint16_t ks_buf[2][kKeys * kKStride];
-    __shared__ __attribute__((aligned(16))) uint16_t vts_buf[2][kD * kVStride];
+// Key-split schedule (SPLIT): the tiles of all (sequence, head, query block)
+// items in a row are dealt to `slots` workgroups in equal contiguous runs, so
+// a launch whose items do not fill the CUs evenly still ends on all of them at
+// once.  A run that covers only part of an item leaves its unnormalised
+// output, row maxima and row sums in the workspace -- entry 2 * slot + 1 when
+// it starts the item, else 2 * slot -- for prefill_merge_kernel.
+constexpr int kPartFloats = kQRows * kD + 2 * kQRows;
 
-    const int g = p.Hq / p.Hk;
-    const int xcd = blockIdx.x % kXcds;
-    const int slot = blockIdx.x / kXcds;
-    const int group = (slot / g) * kXcds + xcd;
-    const int ngroups = p.qblocks * p.B * p.Hk;
-    if (group >= ngroups) return;
-    const int qb = p.qblocks - 1 - group / (p.B * p.Hk);
-    const int rem = group % (p.B * p.Hk);
-    const int b = rem / p.Hk, kvh = rem % p.Hk;
-    const int h = kvh * g + slot % g;
-    const int n = p.seqlens ? max(0, min(p.seqlens[b], p.Nk)) : p.Nk;
+struct PrefillSplit {
+    float* part;
+    int slots, col_tiles;            // tiles of one (sequence, head): its query blocks in order
+    int64_t tiles;                   // B * Hq * col_tiles
+};
 
+// First tile of a slot's run; slots are dealt so that an XCD's slots follow
+// one another (heads of one KV head group meet in one L2).
+__device__ __forceinline__ int64_t slot_begin(const PrefillSplit& sp, int slot) { return slot * sp.tiles / sp.slots; }
+
+__device__ __forceinline__ int query_block_tiles(const PrefillParams& p, int qb) {
+    const int k_end = p.causal ? min(p.Nk, min(qb * kQRows + kQRows, p.Lq) + p.Nk - p.Lq) : p.Nk;
+    return (k_end + kKeys - 1) / kKeys;
+}
+
+// One item's tiles [t0, t1): to the output when they are all of its `whole`
+// tiles, else to the partial entry `part`.
+template <bool SPLIT>
+__device__ __forceinline__ void prefill_item(const PrefillParams& p, int b, int h, int qb, int n, int t0, int t1,
+                                             int whole, float* part, uint16_t (*ks_buf)[kKeys * kKStride],
+                                             uint16_t (*vts_buf)[kD * kVStride]) {
+    const int kvh = h / (p.Hq / p.Hk);
     // the wave index in a scalar register: the full-tile test below is then a
     // scalar branch, and the masked path's index arithmetic stays inside it
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int col = lane & 15, grp = lane >> 4;
     const int q0 = qb * kQRows + wave * 32;
     const int shift = n - p.Lq;
-    int k_end = n;
-    if (p.causal) k_end = min(n, min(qb * kQRows + kQRows, p.Lq) + shift);
-    const int ntiles = k_end > 0 ? (k_end + kKeys - 1) / kKeys : 0;
+    const int ntiles = t1;
 
     // Query RoPE: the rows' positions first, their table pairs once the
     // first K/V tile's loads are issued, the rotation before the tile loop.
@@ -263,22 +276,22 @@ prefill_kernel(PrefillParams p) {
     const uint16_t* vb = p.v + (int64_t)b * p.v_sb + (int64_t)kvh * p.v_sh;
     const TileOffsets toff = tile_offsets(p.k_sn, p.v_sn);
     TileRegs tr;
-    if (ntiles > 0) load_tile(tr, kb, vb, p.k_sn, p.v_sn, 0, n, toff);
+    if (t0 < ntiles) load_tile(tr, kb, vb, p.k_sn, p.v_sn, t0 * kKeys, n, toff);
     if (p.pairs) {
         QPairs qp[2];
 #pragma unroll
         for (int nt = 0; nt < 2; ++nt) load_q_pairs(qp[nt], p.pairs + qpos[nt] * kD, grp, p.repeats);
-        if (ntiles > 0) {
-            store_tile(tr, ks_buf[0], vts_buf[0]);
-            if (ntiles > 1) load_tile(tr, kb, vb, p.k_sn, p.v_sn, kKeys, n, toff);
+        if (t0 < ntiles) {
+            store_tile(tr, ks_buf[t0 & 1], vts_buf[t0 & 1]);
+            if (t0 + 1 < ntiles) load_tile(tr, kb, vb, p.k_sn, p.v_sn, (t0 + 1) * kKeys, n, toff);
         }
 #pragma unroll
         for (int nt = 0; nt < 2; ++nt) rope_q_operand(qr[nt], qp[nt]);
-    } else if (ntiles > 0) {
-        store_tile(tr, ks_buf[0], vts_buf[0]);
-        if (ntiles > 1) load_tile(tr, kb, vb, p.k_sn, p.v_sn, kKeys, n, toff);
+    } else if (t0 < ntiles) {
+        store_tile(tr, ks_buf[t0 & 1], vts_buf[t0 & 1]);
+        if (t0 + 1 < ntiles) load_tile(tr, kb, vb, p.k_sn, p.v_sn, (t0 + 1) * kKeys, n, toff);
     }
-    if (ntiles > 0) __syncthreads();
+    if (t0 < ntiles) __syncthreads();
     // V^T operand offsets: chunk c of row 16 md + col sits at c ^ (2 md + col / 8) % 8
     int vrow[4];
 #pragma unroll
@@ -286,7 +299,7 @@ prefill_kernel(PrefillParams p) {
     // the wave's earliest query sees keys up to q0 + shift
     const int wave_last = p.causal ? q0 + shift : n - 1;
 
-    for (int t = 0; t < ntiles; ++t) {
+    for (int t = t0; t < ntiles; ++t) {
         const int k0 = t * kKeys;
         const uint16_t* ks = ks_buf[t & 1];
         const uint16_t* vts = vts_buf[t & 1];
@@ -378,6 +391,21 @@ prefill_kernel(PrefillParams p) {
         __syncthreads();
     }
 
+    if (SPLIT && (t0 > 0 || t1 < whole)) {
+        // rows 32 wave + 16 nt + col, columns 16 md + 4 grp + [0, 4)
+#pragma unroll
+        for (int nt = 0; nt < 2; ++nt) {
+            const int row = 32 * wave + 16 * nt + col;
+            const float tot = rows_sum(lacc[nt][0]);
+#pragma unroll
+            for (int md = 0; md < 8; ++md) *reinterpret_cast<v4f*>(part + row * kD + 16 * md + 4 * grp) = o[md][nt];
+            if (grp == 0) {
+                part[kQRows * kD + row] = m[nt];
+                part[kQRows * kD + kQRows + row] = tot;
+            }
+        }
+        return;
+    }
 #pragma unroll
     for (int nt = 0; nt < 2; ++nt) {
         const float tot = rows_sum(lacc[nt][0]);
@@ -397,7 +425,126 @@ prefill_kernel(PrefillParams p) {
     }
 }
 
+// Workgroup -> item by XCD-grouped, longest-first order.
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
+prefill_kernel(PrefillParams p) {
+    __shared__ __attribute__((aligned(16))) uint16_t ks_buf[2][kKeys * kKStride];
+    __shared__ __attribute__((aligned(16))) uint16_t vts_buf[2][kD * kVStride];
+    const int g = p.Hq / p.Hk;
+    const int xcd = blockIdx.x % kXcds;
+    const int slot = blockIdx.x / kXcds;
+    const int group = (slot / g) * kXcds + xcd;
+    const int ngroups = p.qblocks * p.B * p.Hk;
+    if (group >= ngroups) return;
+    const int qb = p.qblocks - 1 - group / (p.B * p.Hk);
+    const int rem = group % (p.B * p.Hk);
+    const int b = rem / p.Hk, h = rem % p.Hk * g + slot % g;
+    const int n = p.seqlens ? max(0, min(p.seqlens[b], p.Nk)) : p.Nk;
+    int k_end = n;
+    if (p.causal) k_end = min(n, min(qb * kQRows + kQRows, p.Lq) + n - p.Lq);
+    const int ntiles = k_end > 0 ? (k_end + kKeys - 1) / kKeys : 0;
+    prefill_item<false>(p, b, h, qb, n, 0, ntiles, ntiles, nullptr, ks_buf, vts_buf);
+}
+
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
+prefill_split_kernel(PrefillParams p, PrefillSplit sp) {
+    __shared__ __attribute__((aligned(16))) uint16_t ks_buf[2][kKeys * kKStride];
+    __shared__ __attribute__((aligned(16))) uint16_t vts_buf[2][kD * kVStride];
+    const int slot = (int)(blockIdx.x % kXcds) * (sp.slots / kXcds) + blockIdx.x / kXcds;
+    int64_t pos = slot_begin(sp, slot);
+    const int64_t end = slot_begin(sp, slot + 1);
+    while (pos < end) {
+        const int head = (int)(pos / sp.col_tiles);
+        int t0 = (int)(pos % sp.col_tiles), qb = 0, whole = query_block_tiles(p, 0);
+        while (t0 >= whole) {
+            t0 -= whole;
+            whole = query_block_tiles(p, ++qb);
+        }
+        const int t1 = (int)min<int64_t>(whole, t0 + end - pos);
+        float* part = sp.part + (int64_t)(2 * slot + (t0 == 0)) * kPartFloats;
+        prefill_item<true>(p, head / p.Hq, head % p.Hq, qb, p.Nk, t0, t1, whole, part, ks_buf, vts_buf);
+        pos += t1 - t0;
+    }
+}
+
+// Merges the runs of an item that lies in more than one slot.  A workgroup per
+// (item, 32 rows): eight lanes a row, sixteen columns each.
+__global__ void __launch_bounds__(256)
+prefill_merge_kernel(PrefillParams p, PrefillSplit sp) {
+    const int item = blockIdx.x / 4, quarter = blockIdx.x % 4;
+    const int qb = item % p.qblocks, head = item / p.qblocks;
+    int64_t first = (int64_t)head * sp.col_tiles;
+    for (int i = 0; i < qb; ++i) first += query_block_tiles(p, i);
+    const int64_t last = first + query_block_tiles(p, qb) - 1;
+    // the slots that hold the item's first and last tile
+    auto slot_of = [&](int64_t pos) {
+        int s = (int)(pos * sp.slots / sp.tiles);
+        while (slot_begin(sp, s + 1) <= pos) ++s;
+        return s;
+    };
+    const int s0 = slot_of(first), s1 = slot_of(last);
+    const int row = 32 * quarter + threadIdx.x / 8, c0 = threadIdx.x % 8 * 4;
+    const int qi = qb * kQRows + row;
+    if (s0 == s1 || qi >= p.Lq) return;
+    auto entry = [&](int s) {
+        return sp.part + (int64_t)(2 * s + (s == s0 && slot_begin(sp, s) <= first)) * kPartFloats;
+    };
+    float M = kNegInf;
+    for (int s = s0; s <= s1; ++s) M = fmaxf(M, entry(s)[kQRows * kD + row]);
+    const float base = M == kNegInf ? 0.f : M;
+    float L = 0.f;
+    v4f acc[4] = {};
+    for (int s = s0; s <= s1; ++s) {
+        const float* e = entry(s);
+        const float w = fast_exp2(e[kQRows * kD + row] - base);
+        L += w * e[kQRows * kD + kQRows + row];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[i] += w * *reinterpret_cast<const v4f*>(e + row * kD + 32 * i + c0);
+    }
+    const float inv = L > 0.f ? 1.f / L : 0.f;
+    const int b = head / p.Hq, h = head % p.Hq;
+    uint16_t* dst = p.out + (int64_t)b * p.o_sb + (int64_t)qi * p.o_sl + (int64_t)h * p.o_sh;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        *reinterpret_cast<u32x2*>(dst + 32 * i + c0) =
+            u32x2{pack2(acc[i][0] * inv, acc[i][1] * inv), pack2(acc[i][2] * inv, acc[i][3] * inv)};
+    if (p.lse && threadIdx.x % 8 == 0)
+        p.lse[((int64_t)b * p.Hq + h) * p.Lq + qi] = L > 0.f ? (M + __log2f(L)) * kLn2 : kNegInf;
+}
+
 bool al16(const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15) == 0; }
+
+// The key-split schedule of a call, or slots = 0 where whole items do: the
+// cheaper of two estimates in us, for items that leave CUs idle or unevenly
+// loaded (up to two a CU; beyond that longest-first order evens them out: 1280
+// items of up to 49 tiles 251 whole, 295 split).  A tile of 64 keys takes a
+// workgroup 1.55 us alone on its CU and 2.3 beside another; the partials of
+// the runs and their merge cost about 15 + 0.035 a run.  Whole against split:
+// 320 items of up to 144 tiles 281 / 235 us, 320 of 67 127 / 129, 320 of 36
+// 69 / 77, 400 of 98 201 / 210, 512 of 79 (two a CU exactly) 180 / 207, 160 of
+// 57 91 / 76, 120 of 99 148 / 89.
+PrefillSplit plan_split(const slimkv_prefill_attention_args* a) {
+    PrefillSplit sp{};
+    if (a->seqlens_k || a->keys <= 0 || a->batch <= 0 || a->queries <= 0 || (a->causal && a->keys < a->queries)) return sp;
+    const int64_t qblocks = (a->queries + kQRows - 1) / kQRows;
+    int64_t tiles = 0, longest = 0;
+    for (int64_t qb = 0; qb < qblocks; ++qb) {
+        const int64_t k_end = a->causal ? std::min<int64_t>(a->keys, std::min<int64_t>(qb * kQRows + kQRows, a->queries) + a->keys - a->queries)
+                                        : a->keys;
+        longest = (k_end + kKeys - 1) / kKeys;
+        tiles += longest;
+    }
+    const int cu = device_cu_count(), slots = 2 * cu / kXcds * kXcds;
+    const int64_t items = a->batch * a->heads * qblocks, total = a->batch * a->heads * tiles;
+    if (slots < kXcds || tiles > (1 << 30) || total < slots || items > 2 * cu) return sp;
+    const double whole = longest * (items <= cu ? 1.55 : 1.9 + 0.4 * (double)(items - cu) / cu);
+    const double split = 15 + 0.035 * (double)(slots + items) + 2.3 * (double)total / slots;
+    if (split > 0.93 * whole) return sp;
+    sp.slots = slots;
+    sp.col_tiles = (int)tiles;
+    sp.tiles = total;
+    return sp;
+}
 
 }  // namespace
 
@@ -405,7 +552,9 @@ bool al16(const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15) == 0
 
 using namespace slimkv;
 
-extern "C" int slimkv_prefill_attention(const slimkv_prefill_attention_args* a, void* stream) {
+namespace {
+
+int prefill_run(const slimkv_prefill_attention_args* a, void* workspace, size_t workspace_bytes, void* stream) {
     if (!a || !a->q || !a->k || !a->v || !a->out) return fail(SLIMKV_EINVAL, "null pointer");
     if (a->head_dim != kD) return fail(SLIMKV_EUNSUP, "prefill attention supports head_dim 128");
     if (a->batch < 0 || a->queries < 0 || a->keys < 0 || a->heads <= 0 || a->kv_heads <= 0 ||
@@ -441,9 +590,34 @@ extern "C" int slimkv_prefill_attention(const slimkv_prefill_attention_args* a, 
         p.pairs = a->rope_pairs; p.rope_rows = a->rope_rows; p.repeats = a->rope_repeats ? 1 : 0;
         p.q_pos = a->q_positions; p.qpos_sb = a->qpos_sb;
     }
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    PrefillSplit sp = plan_split(a);
+    if (sp.slots && workspace && workspace_bytes >= (size_t)sp.slots * 2 * kPartFloats * sizeof(float)) {
+        sp.part = static_cast<float*>(workspace);
+        hipLaunchKernelGGL(prefill_split_kernel, dim3(sp.slots), dim3(256), 0, st, p, sp);
+        hipLaunchKernelGGL(prefill_merge_kernel, dim3((unsigned)(4 * p.B * p.Hq * p.qblocks)), dim3(256), 0, st, p, sp);
+        return check_hip(hipGetLastError(), "prefill attention launch");
+    }
     const int64_t groups = (int64_t)p.qblocks * p.B * p.Hk;
     const int64_t grid = (groups + kXcds - 1) / kXcds * kXcds * (p.Hq / p.Hk);
     if (grid > 0x7fffffff) return fail(SLIMKV_EINVAL, "prefill grid too large");
-    hipLaunchKernelGGL(prefill_kernel, dim3((unsigned)grid), dim3(256), 0, static_cast<hipStream_t>(stream), p);
+    hipLaunchKernelGGL(prefill_kernel, dim3((unsigned)grid), dim3(256), 0, st, p);
     return check_hip(hipGetLastError(), "prefill attention launch");
+}
+
+}  // namespace
+
+extern "C" int slimkv_prefill_attention(const slimkv_prefill_attention_args* a, void* stream) {
+    return prefill_run(a, nullptr, 0, stream);
+}
+
+extern "C" size_t slimkv_prefill_attention_workspace(const slimkv_prefill_attention_args* a) {
+    if (!a || a->heads <= 0) return 0;
+    return (size_t)plan_split(a).slots * 2 * kPartFloats * sizeof(float);
+}
+
+extern "C" int slimkv_prefill_attention_split(const slimkv_prefill_attention_args* a, void* workspace,
+                                              size_t workspace_bytes, void* stream) {
+    if (workspace && !al16(workspace)) return fail(SLIMKV_EINVAL, "the workspace must be 16-byte aligned");
+    return prefill_run(a, workspace, workspace_bytes, stream);
 }

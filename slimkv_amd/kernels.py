@@ -123,7 +123,14 @@ def prefill_attention(q, k, v, scale, causal=True, seqlens_k=None, out=None, lse
         _ptr(q), *q.stride()[:3], _ptr(k), *k.stride()[:3], _ptr(v), *v.stride()[:3],
         _ptr(out), *out.stride()[:3], _ptr(lse), _ptr(seqlens_k),
         B, Lq, Hq, Hk, N, D, float(scale), int(bool(causal)), *rope)
-    check(lib().slimkv_prefill_attention(ctypes.byref(a), _lib.stream_handle(q.device)))
+    nbytes = lib().slimkv_prefill_attention_workspace(ctypes.byref(a))
+    ws = None
+    if nbytes:
+        try:
+            ws = _workspace(nbytes, q.device)
+        except torch.OutOfMemoryError:       # the call runs whole without it
+            nbytes = 0
+    check(lib().slimkv_prefill_attention_split(ctypes.byref(a), _ptr(ws), nbytes, _lib.stream_handle(q.device)))
     return out, lse
 
 

@@ -2663,6 +2663,7 @@ struct LatentPlan {
     int wq;               // q_lat width per head
     int parts;
     size_t qrot_off, qlat_off, shift_off, rml_off, racc_off, lml_off, lacc_off, total;
+    size_t bound;         // total under the most splits that this many rows or fewer take, whatever the other sizes
     size_t prologue_lds;
 };
 
@@ -2811,7 +2812,15 @@ int plan_latent(const slimkv_latent_decode_args* a, LatentPlan* p, const PagedRo
     // dense rows do; 64 sequences of U[1K, 128K] tokens ran a step in 0.151 ms
     // at 3.5 per CU, 0.160 at 2.5, 0.164 at 3 and 0.168 at 4 (beacon
     // workgroups first in the grid).
-    int fill_target = cu * 7 / 2;
+    // A split's fixed part (its first pages' round trip, its partial) weighs
+    // more where the rows are few and a sequence is cut often: below 56
+    // sequences (16 splits each) and 704 rows a CU, 2.5 items per CU (32
+    // sequences of U[1K, 64K] tokens at ratio 8, rank 32: 45.7 against 48.6
+    // us a step; 48 of U[1K, 32K] 46.6 against 50.6; 32 of U[1K, 96K],
+    // 198K rows, 71.2 against 69.1; 64 sequences with 135K rows 59.8 against
+    // 58.0).
+    int fill_target = cu * 7 / 2, most_items = fill_target;
+    if (pg && B < 56 && (pg->rows_total > 0 ? pg->rows_total : B * nl) < (int64_t)cu * 704) fill_target = cu * 5 / 2;
     // Keep the latent split count within the fast combine's reach (one latent
     // partial register pass, and one split per combine thread with the raw
     // ones): at small batches the slots would otherwise fill with ever shorter
@@ -2825,23 +2834,48 @@ int plan_latent(const slimkv_latent_decode_args* a, LatentPlan* p, const PagedRo
     if (a->lat_splits <= 0) {
         lat_target = (int)std::min<int64_t>(lat_target, (lat_tiles * fast_cap + kWaves - 1) / kWaves);
         fill_target = (int)std::min<int64_t>(fill_target, (lat_tiles * fast_cap + kWaves - 1) / kWaves);
+        most_items = (int)std::min<int64_t>(most_items, (lat_tiles * fast_cap + kWaves - 1) / kWaves);
     }
     // Whole workgroups per CU: round the split count down, never up.
     int lat_req = a->lat_splits;
     if (lat_req <= 0 && !pg)
         lat_req = (int)std::max<int64_t>(1, std::min<int64_t>(kMaxSplits, (int64_t)lat_target * kWaves / lat_tiles));
     p->lat = plan_segment((int)B, 1, P, cols, (int)nl, span, rv, lat_req, lat_target);
-    p->coupled = 0;
-    if (!bd && !pg && has_lat) {
-        // Coupled bases: workgroups that hold every query row (up to 80) and
-        // one such workgroup a CU.  More than one a CU only adds partials;
-        // fewer splits than tiles of 64 rows keep the merge short.
+    p->coupled = !bd && !pg && has_lat;
+    int most_splits = 0;
+    // Raw: one column tile per KV head over the full head width (the raw set
+    // is sinks + tail + current token).  Splits of two tiles measured 2-4 us
+    // faster a layer than one split per tile (and 1-2 us faster than three):
+    // fewer raw partials and workgroups, with the raw rows still read long
+    // before the latent ones.
+    p->raw = plan_segment((int)B, (int)Hkv, (int)Lq * g, 16, (int)a->raw_keys, (int)D, (int)D, raw_req0, 0);
+    if (p->raw.tiles != 1 || p->raw.ks != 8) return fail(SLIMKV_EUNSUP, "raw tile shape");
+    if (p->coupled)
+        p->raw.nwg = wave_item_groups((int)B, p->raw.splits, (int)Hkv, kCoupledWaves);
+    if (p->coupled) {
+        // Coupled bases: workgroups that hold every query row (up to 80), one
+        // of them or a raw workgroup a CU: a latent workgroup that shares its
+        // CU with a raw one ends some 4 us late, and the launch with it.  So
+        // the splits take the CUs that the raw workgroups leave, and no more
+        // splits than their longest one, in whole tiles of 64 rows, needs
+        // (B8 8192 rows: 26 splits of 5 tiles 32.5 us, 32 of 4 34.7, 22 of 6
+        // 33.6; B1 16384: 128 of 2 23.0, 256 of 1 26.2; B3 5461 rows under 80
+        // query rows: 43 of 2 27.9, 85 of 1 and 2 32.2, 29 of 3 30.0).  Past
+        // a quarter of the CUs in raw workgroups the latent ones take all of
+        // them (B16 8192 rows, 80 raw: 16 splits of 8 tiles 49.9 us, 11 of 12
+        // 53.2; B12 with 204 raw: 47.2 against 56.9).
         const int rows16 = (P + 15) / 16;
         p->groups = (rows16 + 4) / 5;
         p->coupled = std::max(2, (rows16 + p->groups - 1) / p->groups);
         const int tiles = (int)((nl + kTileKeys - 1) / kTileKeys);
         int splits = a->lat_splits;
-        if (splits <= 0) splits = (int)std::max<int64_t>(1, cu / ((int64_t)B * p->groups));
+        most_splits = splits > 0 ? 0 : std::min({std::max(1, cu / ((int)B * p->groups)), tiles, kMaxSplits});
+        if (splits <= 0) {
+            const int free_cus = 4 * p->raw.nwg <= cu ? cu - p->raw.nwg : cu;
+            splits = (int)std::max<int64_t>(1, free_cus / ((int64_t)B * p->groups));
+            const int longest = (tiles + splits - 1) / splits;
+            splits = (tiles + longest - 1) / longest;
+        }
         splits = std::min({splits, tiles, kMaxSplits});
         p->lat.splits = splits;
         p->lat.rows_per_split = 0;
@@ -2851,21 +2885,17 @@ int plan_latent(const slimkv_latent_decode_args* a, LatentPlan* p, const PagedRo
         // Compact schedule: size the splits from the total row count so the
         // non-empty splits of all sequences make about fill_target items.
         const int64_t total = pg->rows_total > 0 ? pg->rows_total : B * nl;
-        int64_t rps = (total + fill_target - 1) / fill_target;
-        rps = std::max<int64_t>(rps, (nl + std::min(kMaxSplits, fast_cap) - 1) / std::min(kMaxSplits, fast_cap));
-        rps = std::max<int64_t>(16, (rps + 15) / 16 * 16);
+        const int64_t shortest = (nl + std::min(kMaxSplits, fast_cap) - 1) / std::min(kMaxSplits, fast_cap);
+        auto rows_for = [&](int64_t items) {
+            const int64_t rows = std::max((total + items - 1) / items, shortest);
+            return std::max<int64_t>(16, (rows + 15) / 16 * 16);
+        };
+        const int64_t rps = rows_for(fill_target), least = rows_for(most_items);
+        most_splits = (int)((nl + least - 1) / least);
         p->lat.rows_per_split = (int)rps;
         p->lat.splits = (int)((nl + rps - 1) / rps);
         p->lat.nwg = wave_item_groups((int)B, p->lat.splits, p->lat.tiles);
     }
-    // Raw: one column tile per KV head over the full head width (the raw set
-    // is sinks + tail + current token).  Splits of two tiles measured 2-4 us
-    // faster a layer than one split per tile (and 1-2 us faster than three):
-    // fewer raw partials and workgroups, with the raw rows still read long
-    // before the latent ones.
-    p->raw = plan_segment((int)B, (int)Hkv, (int)Lq * g, 16, (int)a->raw_keys, (int)D, (int)D, raw_req0, 0);
-    if (p->raw.tiles != 1 || p->raw.ks != 8) return fail(SLIMKV_EUNSUP, "raw tile shape");
-    if (p->coupled) p->raw.nwg = wave_item_groups((int)B, p->raw.splits, (int)Hkv, kCoupledWaves);
     p->wq = rk;
     int parts = 1;
     while (parts < 16 && g * (int)Lq * (p->wq / 8) * parts * 2 <= 256) parts *= 2;
@@ -2882,6 +2912,10 @@ int plan_latent(const slimkv_latent_decode_args* a, LatentPlan* p, const PagedRo
     p->lml_off = off; off = align256(off + lr * 8);
     p->lacc_off = off; off = align256(off + lr * (size_t)rv * 4);
     p->total = off;
+    // A workspace asked for at the largest sizes of a run serves the smaller
+    // ones too, which may take more splits.
+    const size_t more = (size_t)B * Hq * Lq * std::max(0, most_splits - p->lat.splits);
+    p->bound = off + (more ? align256(more * 8) + align256(more * (size_t)rv * 4) : 0);
     return SLIMKV_OK;
 }
 
@@ -2890,7 +2924,7 @@ int plan_latent(const slimkv_latent_decode_args* a, LatentPlan* p, const PagedRo
 extern "C" size_t slimkv_latent_decode_workspace(const slimkv_latent_decode_args* a) {
     LatentPlan p{};
     if (plan_latent(a, &p) != SLIMKV_OK) return 0;
-    return p.total;
+    return p.bound;
 }
 
 namespace {
@@ -3159,7 +3193,7 @@ extern "C" size_t slimkv_paged_latent_decode_workspace(const slimkv_paged_latent
     const PagedRows pg = paged_rows(a);
     LatentPlan p{};
     if (plan_latent(&a->base, &p, &pg) != SLIMKV_OK) return 0;
-    return p.total;
+    return p.bound;
 }
 
 extern "C" int slimkv_paged_latent_decode(const slimkv_paged_latent_decode_args* a, void* workspace,

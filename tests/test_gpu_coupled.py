@@ -136,6 +136,28 @@ def test_two_segments_equal_joined_rows(device, first):
     assert all(torch.equal(x, y) for x, y in zip(parts, joined))
 
 
+# rows either side of a whole number of tiles a split, with few raw workgroups
+# (the splits leave them CUs) and with many (they do not)
+@pytest.mark.parametrize('B,raw,n', [(1, 70, 251 * 64), (1, 70, 251 * 64 + 1), (1, 70, 256 * 64 + 1), (9, 1000, 1793)])
+def test_split_counts(device, B, raw, n):
+    check(layer(device, B, 8, 8, n, raw, 64, 64), f'{n} beacons')
+
+
+def test_strided_and_shared_rows(device):
+    """Row strides past the width and one set of rows for every sequence give
+    the bits of contiguous copies."""
+    from slimkv_amd import kernels
+    args, kw, *_ = layer(device, 3, 32, 8, 700, 37, 200, 256, 1, True)
+    q, rk, rv, lk, lv, *rest = args
+    wide_k, wide_v = (torch.cat([t, torch.full_like(t[..., :24], float('nan'))], -1) for t in (lk, lv))
+    want = kernels.latent_decode(*args, **kw)
+    got = kernels.latent_decode(q, rk, rv, wide_k[..., :200], wide_v[..., :256], *rest, **kw)
+    assert all(torch.equal(x, y) for x, y in zip(got, want))
+    shared = kernels.latent_decode(q, rk, rv, lk[:1].expand(3, -1, -1), lv[:1].expand(3, -1, -1), *rest, **kw)
+    copied = kernels.latent_decode(q, rk, rv, lk[:1].repeat(3, 1, 1), lv[:1].repeat(3, 1, 1), *rest, **kw)
+    assert all(torch.equal(x, y) for x, y in zip(shared, copied))
+
+
 def test_device_scratch_holds_fewer_splits(device):
     """The allocation-free call has a fixed scratch: 80 query rows of width 384
     plan more partials than it holds, and then take fewer splits."""
@@ -143,8 +165,8 @@ def test_device_scratch_holds_fewer_splits(device):
     from slimkv_amd import _lib, kernels
     args, kw, out, lse, atol = layer(device, 1, 40, 8, 17000, 1800, 384, 384, 2)
     a, got, got_lse, keep = kernels._latent_args(
-        *args, kw['up_k_bias'], kw['up_v_bias'], False, True, kw['q_positions'], kw['cos'], kw['sin'], None, None, 0, 0,
-        None, None)
+        *args, kw['up_k_bias'], kw['up_v_bias'], False, True, kw['q_positions'], kw['cos'], kw['sin'], None, None, 0,
+        256, None, None)
     assert _lib.lib().slimkv_latent_decode_workspace(ctypes.byref(a)) > 32 << 20
     _lib.check(_lib.lib().slimkv_latent_decode_noalloc(ctypes.byref(a), _lib.stream_handle(device)))
     torch.cuda.synchronize()

@@ -158,6 +158,8 @@ typedef struct slimkv_latent_decode_args {
     int64_t lat_split;
 } slimkv_latent_decode_args;
 
+/* Enough for the call as described and, on bases without blocks, for one with
+ * fewer beacons (whose automatic splits can be more). */
 size_t slimkv_latent_decode_workspace(const slimkv_latent_decode_args* a);
 int slimkv_latent_decode(const slimkv_latent_decode_args* a, void* workspace,
                          size_t workspace_bytes, void* stream);
@@ -263,8 +265,9 @@ typedef struct slimkv_reconstruct_args {
 
 int slimkv_reconstruct(const slimkv_reconstruct_args* a, void* stream);
 
-/* Two reconstructions in one launch where both take the streaming kernel (a
- * contracted latent width up to 64) at the same width -- the K and the V
+/* Two reconstructions in one launch where both contract the same latent width,
+ * up to 64 (streamed) or 128 to 512 (for those at most the first with RoPE,
+ * rows on 16-byte boundaries) -- the K and the V
  * rebuild of one set of beacon rows -- else in two launches; the results are
  * those of two slimkv_reconstruct calls, bit for bit.  The reference runs the
  * K and V up-projections of ReconstructionCache.materialize as two nn.Linear

@@ -9,7 +9,8 @@
 // W (per-KV-head bases, `blocks` diagonal blocks) contracts each output block
 // over its own K block only.
 //
-// One wavefront computes C^T[n, m] = W[n, :] . x[m, :] for 16 outputs x 64
+// Weights without blocks: down_tile_kernel below.  Block-diagonal ones: one
+// wavefront computes C^T[n, m] = W[n, :] . x[m, :] for 16 outputs x 64
 // rows: A = W rows and B = x rows are both contiguous along the contraction,
 // and a lane ends with 4 consecutive outputs of one row (8-byte stores).  Long
 // contractions are split over workgroups into fp32 partials summed in a fixed

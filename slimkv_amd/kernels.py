@@ -499,9 +499,9 @@ def reconstruct(latent, weight, bias=None, *, kv_heads, out=None, dst_rows=None,
 
 
 def reconstruct_pair(first, second):
-    """Two reconstructions in one launch where the library can (both on its
-    streaming kernel at one latent width, as the K and V rebuild of a
-    window's beacon rows are), the same bits as two reconstruct calls.
+    """Two reconstructions in one launch where the library can (one
+    latent width, as the K and V rebuild of a window's beacon rows have), the
+    same bits as two reconstruct calls.
     `first` / `second`: dicts of reconstruct's arguments.  Returns the two
     outputs."""
     a, out_a, keep_a = _reconstruct_args(**_recon_kwargs(first))

@@ -143,6 +143,14 @@ def test_split_counts(device, B, raw, n):
     check(layer(device, B, 8, 8, n, raw, 64, 64), f'{n} beacons')
 
 
+def test_workspace_of_more_beacons_serves_fewer(device):
+    """252 tiles of 64 rows take 126 splits, 251 tiles 251."""
+    from slimkv_amd import kernels
+    few, many = (kernels.latent_decode_workspace_bytes(*layer(device, 1, 8, 8, n * 64, 5, 64, 64)[0])
+                 for n in (251, 252))
+    assert few <= many
+
+
 def test_strided_and_shared_rows(device):
     """Row strides past the width and one set of rows for every sequence give
     the bits of contiguous copies."""

@@ -3301,8 +3301,13 @@ int plan_recon(const slimkv_recon_decode_args* r, ReconPlan* p) {
         // recon_split_kernel: a workgroup per (b, group of kWaves KV heads, split)
         p->rec.nwg = (int)(groups * p->rec.splits);
     } else {
+        // One and a half workgroups of rebuilt rows a CU, so that the resident
+        // slots (two a CU) hold the raw workgroups too: filled with rebuilt
+        // rows alone, the launch ends a round later (B2 4096 rows of 32/8
+        // heads: 42.8 us the layer against 46.4 at two a CU, 44.2 at one; B1
+        // 8192 44.3, 48.0, 44.9; B8 4096 127.3, 128.9, 128.6).
         p->rec = plan_segment((int)B, (int)Hkv, (int)Lq * g, 16, nl, (int)D, (int)D, a->lat_splits,
-                              cu * split_occupancy(8, 8));
+                              cu * 3 / 2);
     }
     size_t off = 0;
     p->v_latent = (p->fused || recon_v_latent(a)) ? 1 : 0;

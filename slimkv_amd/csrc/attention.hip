@@ -2504,20 +2504,19 @@ hipError_t dispatch_split(int ka, int kb, const SplitParams& prm, int grid, hipS
 }
 
 // Resident workgroups per CU of a split-kernel instance (cached per device).
-int split_occupancy(int ka, int kb) {
+int split_occupancy(int ka) {
     static std::mutex mu;
     static std::vector<std::pair<int, int>> keys;
     static std::vector<int> vals;
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) dev = 0;
-    const int key = (dev << 16) | (ka << 8) | kb;
+    const int key = (dev << 16) | ka;
     std::lock_guard<std::mutex> lock(mu);
     for (size_t i = 0; i < keys.size(); ++i)
         if (keys[i].first == key) return vals[i];
     const void* fn = nullptr;
-#define SLIMKV_FN(A, B) if (ka == A && kb == B) fn = reinterpret_cast<const void*>(&split_kernel<A, B>);
-    SLIMKV_FN(2, 0) SLIMKV_FN(2, 8) SLIMKV_FN(4, 0) SLIMKV_FN(6, 0) SLIMKV_FN(8, 0) SLIMKV_FN(12, 0) SLIMKV_FN(16, 0) SLIMKV_FN(24, 0)
-    SLIMKV_FN(4, 8) SLIMKV_FN(6, 8) SLIMKV_FN(8, 8) SLIMKV_FN(12, 8) SLIMKV_FN(16, 8) SLIMKV_FN(24, 8)
+#define SLIMKV_FN(A) if (ka == A) fn = reinterpret_cast<const void*>(&split_kernel<A, 0>);
+    SLIMKV_FN(2) SLIMKV_FN(4) SLIMKV_FN(6) SLIMKV_FN(8) SLIMKV_FN(12) SLIMKV_FN(16) SLIMKV_FN(24)
 #undef SLIMKV_FN
     int blocks = 0;
     if (!fn || hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, fn, kThreads, 0) != hipSuccess || blocks < 1)
@@ -2551,7 +2550,7 @@ int plan_attention(const slimkv_attention_args* a, AttnPlan* plan) {
     const int span = (int)std::max(a->width_k, a->width_v);
     const int ks = round_even_tile(span);
     if (ks < 0) return fail(SLIMKV_EUNSUP, "width not supported");
-    const int target = device_cu_count() * split_occupancy(ks, 0);
+    const int target = device_cu_count() * split_occupancy(ks);
     plan->sp = plan_segment((int)B, (int)Hk, P, 16, (int)N, span, (int)a->width_v, a->splits, target);
     if (a->splits > kMaxSplits) return fail(SLIMKV_EINVAL, "too many splits");
     const size_t rows = (size_t)B * Hq * Lq * plan->sp.splits;

@@ -49,12 +49,20 @@ def _flat_latents(latent):
     return latent.transpose(1, 2).reshape(batch, length, heads * dim)
 
 
+def _differentiated(part):
+    """Whether torch's copy of `part` would record a gradient or carry a
+    forward-mode tangent."""
+    return (part.requires_grad and torch.is_grad_enabled()) or torch.autograd.forward_ad.unpack_dual(part).tangent is not None
+
+
 def _copyable(part, out):
-    """Whether a full-width part can be copied as rows: out's type, device,
-    batch and heads, 16-byte rows, no gradient to record."""
-    return (not (part.requires_grad and torch.is_grad_enabled()) and part.dtype == out.dtype == torch.bfloat16 and part.device == out.device
-            and part.shape[:2] == out.shape[:2] and part.shape[3] == out.shape[3] and part.stride(3) == 1 and part.data_ptr() % 16 == 0
-            and not any(s % 8 for s in part.stride()[:3]))
+    """Whether a full-width part can be copied as rows: plain memory of out's
+    type, device, batch and heads, 16-byte rows, no derivative to carry."""
+    if type(part) not in (torch.Tensor, torch.nn.Parameter) or part.is_neg() or _differentiated(part):
+        return False
+    return (part.dtype == out.dtype == torch.bfloat16 and part.device == out.device
+            and part.shape[:2] == out.shape[:2] and part.shape[3] == out.shape[3] and part.stride(3) == 1
+            and part.data_ptr() % 16 == 0 and not any(s % 8 for s in part.stride()[:3]))
 
 
 class ReconstructionCache:
@@ -88,11 +96,11 @@ class ReconstructionCache:
         bd = is_block_diagonal(up.weight, heads)
         if self.history is not None and n_hist and self.window is None:
             # the whole set in one call where the row copies take the parts as they are
-            rows = [(row, t) for row, t in ((0, self.sink), (n_sink + n_hist, self.raw), (total - _length(current), current))
-                    if t is not None and t.shape[2]]
+            parts = ((0, self.sink), (n_sink + n_hist, self.raw), (total - _length(current), current))
+            rows = [(row, t) for row, t in parts if t is not None and t.shape[2]]
             if rows and dim == 128 and all(_copyable(t, out) for _, t in rows):
-                return kernels.reconstruct_with_rows(_flat_latents(self.history), up.weight, up.bias, out, n_sink, rows,
-                                                     block_diagonal=bd)
+                return kernels.reconstruct_with_rows(_flat_latents(self.history), up.weight, up.bias, out, n_sink,
+                                                     rows, block_diagonal=bd)
         if self.sink is not None:
             out[:, :, :n_sink] = self.sink
         if self.history is not None:

@@ -139,3 +139,24 @@ def test_prefill_history_follows_the_memory():
         store.append(att, torch.zeros(2, 29, 64), torch.zeros(2, 29, 64), sink_size=4)
     assert store.history == 8
     assert store.follows(empty, empty) and (store.sink, store.history) == (0, 0)
+
+
+@pytest.mark.parametrize('kind', ['plain', 'gradient', 'tangent', 'negative view', 'subclass'])
+def test_rows_copied_as_bytes_are_plain_ones(kind):
+    """A cache part is copied as raw rows only where its bytes are all a torch
+    copy would carry over."""
+    from slimkv_amd.memory import _copyable
+
+    class Wrapped(torch.Tensor):
+        pass
+    out = torch.empty(1, 2, 9, 128, dtype=torch.bfloat16)
+    part = torch.zeros(1, 2, 4, 128, dtype=torch.bfloat16)
+    with torch.autograd.forward_ad.dual_level():
+        part = {'plain': lambda: part, 'gradient': lambda: part.requires_grad_(),
+                'tangent': lambda: torch.autograd.forward_ad.make_dual(part, torch.ones_like(part)),
+                'negative view': lambda: torch._neg_view(part),
+                'subclass': lambda: part.as_subclass(Wrapped)}[kind]()
+        assert _copyable(part, out) == (kind == 'plain')
+    if kind == 'gradient':
+        with torch.no_grad():
+            assert _copyable(part, out)

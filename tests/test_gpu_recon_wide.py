@@ -97,3 +97,23 @@ def test_rows_around_a_rebuilt_history(device, rank, per_head, B, sink, n, raw, 
         shifted = torch.empty(parts[2].numel() + 1, dtype=torch.bfloat16, device=device)[1:].view(parts[2].shape)
         shifted.copy_(parts[2])
         assert torch.equal(cache.materialize(attention, shifted), want)
+
+
+def test_forward_mode_reaches_the_rows_around_a_history(device):
+    """The tangents of sink and current rows are carried into the whole set, as
+    torch's copies of them carry it."""
+    from types import SimpleNamespace
+    from torch.autograd import forward_ad
+    from slimkv_amd.memory import ReconstructionCache
+    gen = torch.Generator(device=device).manual_seed(9)
+    up = torch.nn.Linear(256, HKV * D, bias=False, device=device, dtype=torch.bfloat16).requires_grad_(False)
+    sink, current, dsink, dcurrent = (torch.randn(1, HKV, n, D, generator=gen, device=device).to(torch.bfloat16)
+                                      for n in (4, 7, 4, 7))
+    latent = torch.randn(1, 1, 20, 256, generator=gen, device=device).to(torch.bfloat16)
+    attention = SimpleNamespace(beacon_k_up_proj=up, num_key_value_heads=HKV, head_dim=D)
+    plain = ReconstructionCache(sink, latent, None, None, None, HKV, D, 'k').materialize(attention, current)
+    with forward_ad.dual_level():
+        cache = ReconstructionCache(forward_ad.make_dual(sink, dsink), latent, None, None, None, HKV, D, 'k')
+        got, tangent = forward_ad.unpack_dual(cache.materialize(attention, forward_ad.make_dual(current, dcurrent)))
+    assert torch.equal(got, plain)
+    assert torch.equal(tangent, torch.cat([dsink, torch.zeros_like(tangent[:, :, 4:24]), dcurrent], 2))

@@ -366,10 +366,10 @@ def check(code):
 
 
 def stream_handle(device):
-    """Address of torch's current stream on `device` (a torch.device or what
-    torch.device takes), without building a Stream object for it."""
+    """Address of torch's current stream on `device` (what
+    torch.cuda.current_stream takes); a tensor's device is looked up without
+    building a Stream object for it."""
     import torch
-    if not isinstance(device, torch.device):
-        device = torch.device(device)
-    index = torch.cuda.current_device() if device.index is None else device.index
-    return torch._C._cuda_getCurrentRawStream(index)
+    if isinstance(device, torch.device) and device.type == 'cuda' and device.index is not None:
+        return torch._C._cuda_getCurrentRawStream(device.index)
+    return torch.cuda.current_stream(device).cuda_stream

@@ -94,3 +94,17 @@ def test_errors_are_reported_without_a_gpu():
     assert b'null' in _lib.lib().slimkv_last_error()
     with pytest.raises(ValueError):
         _lib.check(-1)
+
+
+@pytest.mark.gpu
+def test_stream_handle_takes_what_current_stream_takes(device):
+    import torch
+    from slimkv_amd import _lib
+    side = torch.cuda.Stream(device)
+    with torch.cuda.stream(side):
+        for named in (device, 'cuda', 'cuda:0', 0, None, torch.device('cuda')):
+            assert _lib.stream_handle(named) == side.cuda_stream
+    assert _lib.stream_handle(device) == torch.cuda.current_stream(device).cuda_stream
+    for other in ('cpu', torch.device('cpu'), 'meta'):
+        with pytest.raises(ValueError):
+            _lib.stream_handle(other)

@@ -1526,20 +1526,17 @@ __device__ __forceinline__ float wave_first(float v) {
 // KV heads, rebuilt full-width rows, plain attention at any width).  It is
 // bound by memory round trips, so the loads that depend on nothing are issued
 // first (U_V pieces, the first partials of each segment, one split's
-// statistics a thread) and the rest by 1024 threads side by side: a thread
+// statistics a thread) and the rest by T threads side by side: a thread
 // owns one four-column quad of every T / quads-th split, and eight
 // neighbouring lanes share a row of U_V, reading its pieces as whole cache
-// lines.  A serial loop over splits and U_V columns on 128 threads took
-// 46.5 us for 32 rows of 256 latent splits of width 256 (one sequence, now
-// 10.0), 12.7 for 256 rows of 32 splits (7.4) and 13.9 for 64 rows over
-// rebuilt rows (6.8); 512 threads with twice the loads ahead the same.
-constexpr int kWideThreads = 1024;
+// lines.  combine_threads chooses T.
 constexpr int kWideLift = 6;         // U_V pieces a lane: latent widths up to 384
 constexpr int kWideAhead = 4;        // latent quads a thread issues before the statistics (raw: half)
 
-__global__ void __launch_bounds__(kWideThreads)
+template <int T>
+__global__ void __launch_bounds__(T)
 combine_kernel(CombineParams cp) {
-    constexpr int T = kWideThreads, NW = T / 64;
+    constexpr int NW = T / 64;
     __shared__ float wts[2 * kMaxSplits];
     __shared__ float4 part[2][T];            // quad sums of the latent and the raw segment by split group
     __shared__ float accb[kMaxLatW];
@@ -1578,7 +1575,7 @@ combine_kernel(CombineParams cp) {
         const int sp = sb + i * gb;
         fb[i] = bacc[inb && sp < bsp ? sp * bq + kb : 0];
     }
-    const int d8 = t / 8, piece = t % 8;                    // output d8 (T / 8 = 128 at a time)
+    const int d8 = t / 8, piece = t % 8;                    // output d8 (T / 8 at a time)
     u32x4 w[kWideLift];
     const uint16_t* wrow = lift ? cp.up_v + (cp.blockdiag ? h * cp.b_w : 0) : nullptr;
     auto lift_load = [&](int d) {
@@ -1592,7 +1589,7 @@ combine_kernel(CombineParams cp) {
     if (lift) lift_load(min(d8, cp.D - 1));
     const float shift = (cp.b_splits && cp.b_shift) ? cp.b_shift[row] * kLog2e : 0.f;
 
-    // Split maxima and masses: at most 2 * kMaxSplits <= T splits, one a thread.
+    // Split maxima and masses, one split a thread (combine_threads).
     float mv = kNegInf, lv = 0.f;
     if (t < cp.a_splits) {
         mv = aml[2 * t];
@@ -2041,6 +2038,40 @@ bool combine_wave_ok(const CombineParams& cp) {
     return (cp.b_splits + ngr - 1) / ngr <= kWaveLat;
 }
 
+// Threads of the general combine: at least one a split and one a quad of the
+// wider segment (widths up to 384: 96 quads).  Few rows want many
+// threads for each row's round trips, many rows want small workgroups, of which
+// a CU holds more at a time; the lift of a latent accumulator is the longer
+// part and wants more threads.  Times at 128 / 256 / 512 / 1024 threads in us,
+// width 256 with a lift, 16 latent splits and 5 raw: 32 rows 9.4 / 7.2 / 6.0 /
+// 6.8, 512 rows 10.3 / 8.1 / 7.8 / 12.2, 1024 rows 10.7 / 9.7 / 12.3 / 22.5,
+// 4096 rows 26.7 / 27.1 / 36.4 / 84.3; rebuilt rows (no lift) in 12 splits:
+// 256 rows 4.5 / 4.5 / 4.9 / 6.3, 4096 rows 11.3 / 14.0 / 24.4 / 71.1.  Few
+// rows with five quads of partials or more a thread of 512 take 1024 threads,
+// as the partials come from other dies' caches: the layer of four sequences of
+// 4096 rows of width 384 (32 splits) 21.9 against 21.0, of one of 16384 rows
+// (128 splits) 23.1 against 22.3, of three of 5461 rows of widths 320 and 200
+// (43 splits, 17 raw) 28.3 against 27.8; of four of 4096 rows of width 256 (32
+// splits, 4.3 quads) 21.4 against 21.8.
+int combine_threads(const CombineParams& cp, int rows) {
+    const int cu = device_cu_count();
+    const bool lift = cp.b_splits && cp.up_v;
+    if (lift && rows <= cu && cp.a_splits * (cp.a_w / 4) + cp.b_splits * (cp.b_w / 4) >= 5 * 512) return 1024;
+    const int most = lift ? 512 : 256;
+    const int threads = rows <= 2 * cu ? most : (rows <= 4 * cu ? most / 2 : 128);
+    const int splits = cp.a_splits + cp.b_splits;       // at most 2 * kMaxSplits
+    return std::max(threads, splits > 256 ? 512 : (splits > 128 ? 256 : 128));
+}
+
+void launch_combine_general(const CombineParams& cp, int rows, hipStream_t st) {
+    switch (combine_threads(cp, rows)) {
+        case 128: hipLaunchKernelGGL(combine_kernel<128>, dim3(rows), dim3(128), 0, st, cp); break;
+        case 256: hipLaunchKernelGGL(combine_kernel<256>, dim3(rows), dim3(256), 0, st, cp); break;
+        case 512: hipLaunchKernelGGL(combine_kernel<512>, dim3(rows), dim3(512), 0, st, cp); break;
+        default: hipLaunchKernelGGL(combine_kernel<1024>, dim3(rows), dim3(1024), 0, st, cp); break;
+    }
+}
+
 // The one-wave combine takes the shapes it fits (the batch-16 32K decode
 // sweep: 1.180 -> 1.138 ms; the 64-sequence paged step: 0.151 -> 0.147 ms
 // against combine_fast_kernel<128>); more splits or wider latents keep the
@@ -2058,7 +2089,7 @@ void launch_combine(const CombineParams& cp, int rows, hipStream_t st) {
     else if (combine_fast_ok(cp, 256))
         hipLaunchKernelGGL(combine_fast_kernel<256>, dim3(rows), dim3(256), 0, st, cp);
     else
-        hipLaunchKernelGGL(combine_kernel, dim3(rows), dim3(kWideThreads), 0, st, cp);
+        launch_combine_general(cp, rows, st);
 }
 
 // ---------------------------------------------------------------------------

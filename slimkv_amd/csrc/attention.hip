@@ -2810,8 +2810,8 @@ int plan_latent(const slimkv_latent_decode_args* a, LatentPlan* p, const PagedRo
     // times (rank 32: 51.1 against 34.1 us); a group of eight, or four with
     // two queries, one head a tile (ranks 32 / 48: 40.0 / 68.4 against 34.9 /
     // 51.6 us); a group of two, four heads a tile (ranks 16 / 32 / 48: 26.9 /
-    // 36.9 / 55.6 against 22.7 / 32.9 / 48.3 us).  General bases: eight query
-    // rows a tile, every tile reads whole rows.
+    // 36.9 / 55.6 against 22.7 / 32.9 / 48.3 us).  Coupled bases that stay with
+    // the split kernel: eight query rows a tile, every tile reads whole rows.
     int cols = 8;
     if (bd) {
         int heads = std::max(1, std::min(std::max(rk, rv) <= 16 ? 4 : 2, kMaxRows / (g * (int)Lq)));
@@ -2871,7 +2871,20 @@ int plan_latent(const slimkv_latent_decode_args* a, LatentPlan* p, const PagedRo
     if (lat_req <= 0 && !pg)
         lat_req = (int)std::max<int64_t>(1, std::min<int64_t>(kMaxSplits, (int64_t)lat_target * kWaves / lat_tiles));
     p->lat = plan_segment((int)B, 1, P, cols, (int)nl, span, rv, lat_req, lat_target);
-    p->coupled = !bd && !pg && has_lat;
+    // Coupled bases take the coupled kernel, but for few query rows over narrow
+    // latents: one or two of the split kernel's waves hold all of them, read
+    // each row as rarely, and wait for no barrier, while a tile of 64 narrow
+    // rows takes the coupled kernel's eight waves as long as one of wide rows
+    // (the layer, split against coupled, us: 8 rows and width 64, B16 16384 rows
+    // 25.0 / 33.6, B64 4096 rows 31.1 / 45.0, B16 256 rows 13.7 / 14.3; 16 rows
+    // B64 4096 39.9 / 46.8, B1 16384 15.8 / 14.9; 32 rows B16 16384 46.5 / 36.2;
+    // 8 rows with long runs of tiles, width 128: B64 4096 50.7 / 54.5, B16 16384
+    // 36.3 / 38.9, B64 1024 33.3 / 32.7; width 256: B64 4096 79.9 / 87.0, B16
+    // 16384 63.0 / 60.2; width 384 140 / 107).
+    const int tiles64 = (int)((nl + kTileKeys - 1) / kTileKeys), width = (int)std::max(Rk, Rv);
+    const bool narrow = (P <= 16 && width <= 64 && B >= 16) ||
+                        (P <= 8 && B * tiles64 >= 16 * cu && (width <= 128 || (width <= 256 && 4 * B >= cu)));
+    p->coupled = !bd && !pg && has_lat && !narrow;
     int most_splits = 0;
     // Raw: one column tile per KV head over the full head width (the raw set
     // is sinks + tail + current token).  Splits of two tiles measured 2-4 us
@@ -2897,16 +2910,15 @@ int plan_latent(const slimkv_latent_decode_args* a, LatentPlan* p, const PagedRo
         const int rows16 = (P + 15) / 16;
         p->groups = (rows16 + 4) / 5;
         p->coupled = std::max(2, (rows16 + p->groups - 1) / p->groups);
-        const int tiles = (int)((nl + kTileKeys - 1) / kTileKeys);
         int splits = a->lat_splits;
-        most_splits = splits > 0 ? 0 : std::min({std::max(1, cu / ((int)B * p->groups)), tiles, kMaxSplits});
+        most_splits = splits > 0 ? 0 : std::min({std::max(1, cu / ((int)B * p->groups)), tiles64, kMaxSplits});
         if (splits <= 0) {
             const int free_cus = 4 * p->raw.nwg <= cu ? cu - p->raw.nwg : cu;
             splits = (int)std::max<int64_t>(1, free_cus / ((int64_t)B * p->groups));
-            const int longest = (tiles + splits - 1) / splits;
-            splits = (tiles + longest - 1) / longest;
+            const int longest = (tiles64 + splits - 1) / splits;
+            splits = (tiles64 + longest - 1) / longest;
         }
-        splits = std::min({splits, tiles, kMaxSplits});
+        splits = std::min({splits, tiles64, kMaxSplits});
         p->lat.splits = splits;
         p->lat.rows_per_split = 0;
         p->lat.nwg = (int)B * splits * p->groups;

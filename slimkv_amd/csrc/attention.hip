@@ -2848,9 +2848,14 @@ int plan_latent(const slimkv_latent_decode_args* a, LatentPlan* p, const PagedRo
     // sequences of U[1K, 64K] tokens at ratio 8, rank 32: 45.7 against 48.6
     // us a step; 48 of U[1K, 32K] 46.6 against 50.6; 32 of U[1K, 96K],
     // 198K rows, 71.2 against 69.1; 64 sequences with 135K rows 59.8 against
-    // 58.0).
+    // 58.0).  That holds where a sequence's tiles fill a workgroup: with fewer
+    // (rank 16, whose tiles hold four heads) an item is fewer waves, and fewer
+    // items leave the CUs short of loads (16 sequences of up to 16384 beacons
+    // 34.4 against 30.5 us, 32 of up to 8192 33.3 against 29.5).
     int fill_target = cu * 7 / 2, most_items = fill_target;
-    if (pg && B < 56 && (pg->rows_total > 0 ? pg->rows_total : B * nl) < (int64_t)cu * 704) fill_target = cu * 5 / 2;
+    if (pg && B < 56 && (P + cols - 1) / cols >= kWaves &&
+        (pg->rows_total > 0 ? pg->rows_total : B * nl) < (int64_t)cu * 704)
+        fill_target = cu * 5 / 2;
     // Keep the latent split count within the fast combine's reach (one latent
     // partial register pass, and one split per combine thread with the raw
     // ones): at small batches the slots would otherwise fill with ever shorter

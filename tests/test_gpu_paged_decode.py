@@ -119,15 +119,16 @@ def test_compact_schedule_matches_oracle(device, rows_total, layout_args):
         np.testing.assert_allclose(to_np(lse)[b:b + 1], ref_lse, atol=2e-3, rtol=1e-4)
 
 
+@pytest.mark.parametrize('rank', [256, 128])
 @pytest.mark.parametrize('sequences', [55, 56])
 @pytest.mark.parametrize('rows_total', [0, 704 * 256 - 1, 704 * 256])
-def test_split_sizes_either_side_of_their_rule(device, sequences, rows_total):
-    """Fewer, longer splits for few sequences with few rows: the automatic
-    splits against one split of every sequence, within the bf16 of a result
-    and the fp32 of its sums."""
+def test_split_sizes_either_side_of_their_rule(device, sequences, rows_total, rank):
+    """Fewer, longer splits for few sequences with few rows of rank 32 a head:
+    the automatic splits against one split of every sequence, within the bf16
+    of a result and the fp32 of its sums."""
     from slimkv_amd import kernels
     lengths = [(37 * i) % 400 for i in range(sequences - 1)] + [1500]
-    c = _case(device, (16, 8, 256, 256, 1024), lengths, [1 + i % 70 for i in range(sequences)], seed=sequences)
+    c = _case(device, (16, 8, rank, rank, 1024), lengths, [1 + i % 70 for i in range(sequences)], seed=sequences)
     got, want = (kernels.paged_latent_decode(
         c['q'], c['raw_k'], c['raw_v'], c['pages'], c['tables'], c['lengths'], c['lat_keys'], c['layout'], c['up_k'],
         c['up_v'], D ** -0.5, rows_total=rows_total, block_diagonal=True, raw_lengths=c['raw_lengths'], lat_splits=n)

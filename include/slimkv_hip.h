@@ -158,8 +158,8 @@ typedef struct slimkv_latent_decode_args {
     int64_t lat_split;
 } slimkv_latent_decode_args;
 
-/* Enough for the call as described and, on bases without blocks, for one with
- * fewer beacons (whose automatic splits can be more). */
+/* Enough for the call as described and, on bases without blocks and with
+ * automatic splits, for one with fewer beacons (whose splits can be more). */
 size_t slimkv_latent_decode_workspace(const slimkv_latent_decode_args* a);
 int slimkv_latent_decode(const slimkv_latent_decode_args* a, void* workspace,
                          size_t workspace_bytes, void* stream);
@@ -224,6 +224,8 @@ typedef struct slimkv_paged_latent_decode_args {
     const int64_t* raw_table; int64_t raw_t_sb, raw_t_cols;
 } slimkv_paged_latent_decode_args;
 
+/* Enough for the call as described and for one with a larger rows_total (a
+ * smaller one takes shorter splits and can need more). */
 size_t slimkv_paged_latent_decode_workspace(const slimkv_paged_latent_decode_args* a);
 int slimkv_paged_latent_decode(const slimkv_paged_latent_decode_args* a, void* workspace,
                                size_t workspace_bytes, void* stream);

@@ -2693,7 +2693,7 @@ struct LatentPlan {
     int wq;               // q_lat width per head
     int parts;
     size_t qrot_off, qlat_off, shift_off, rml_off, racc_off, lml_off, lacc_off, total;
-    size_t bound;         // total under the most splits that this many rows or fewer take, whatever the other sizes
+    size_t bound;         // workspace asked for: total, or more where the header promises it for other sizes
     size_t prologue_lds;
 };
 
@@ -2890,7 +2890,10 @@ int plan_latent(const slimkv_latent_decode_args* a, LatentPlan* p, const PagedRo
     const bool narrow = (P <= 16 && width <= 64 && B >= 16) ||
                         (P <= 8 && B * tiles64 >= 16 * cu && (width <= 128 || (width <= 256 && 4 * B >= cu)));
     p->coupled = !bd && !pg && has_lat && !narrow;
-    int most_splits = 0;
+    // most automatic splits of the calls that a workspace asked for here must
+    // serve: bases without blocks, fewer beacons (few rows may take the split
+    // kernel)
+    int most_splits = bd || pg || P > 16 || a->lat_splits > 0 ? 0 : (int)std::min<int64_t>(lat_req, (nl + 15) / 16);
     // Raw: one column tile per KV head over the full head width (the raw set
     // is sinks + tail + current token).  Splits of two tiles measured 2-4 us
     // faster a layer than one split per tile (and 1-2 us faster than three):
@@ -2916,8 +2919,8 @@ int plan_latent(const slimkv_latent_decode_args* a, LatentPlan* p, const PagedRo
         p->groups = (rows16 + 4) / 5;
         p->coupled = std::max(2, (rows16 + p->groups - 1) / p->groups);
         int splits = a->lat_splits;
-        most_splits = splits > 0 ? 0 : std::min({std::max(1, cu / ((int)B * p->groups)), tiles64, kMaxSplits});
         if (splits <= 0) {
+            most_splits = std::max(most_splits, std::min({std::max(1, cu / ((int)B * p->groups)), tiles64, kMaxSplits}));
             const int free_cus = 4 * p->raw.nwg <= cu ? cu - p->raw.nwg : cu;
             splits = (int)std::max<int64_t>(1, free_cus / ((int64_t)B * p->groups));
             const int longest = (tiles64 + splits - 1) / splits;
@@ -2933,12 +2936,16 @@ int plan_latent(const slimkv_latent_decode_args* a, LatentPlan* p, const PagedRo
         // non-empty splits of all sequences make about fill_target items.
         const int64_t total = pg->rows_total > 0 ? pg->rows_total : B * nl;
         const int64_t shortest = (nl + std::min(kMaxSplits, fast_cap) - 1) / std::min(kMaxSplits, fast_cap);
-        auto rows_for = [&](int64_t items) {
-            const int64_t rows = std::max((total + items - 1) / items, shortest);
+        auto rows_for = [&](int64_t rows_total, int64_t items) {
+            const int64_t rows = std::max((rows_total + items - 1) / items, shortest);
             return std::max<int64_t>(16, (rows + 15) / 16 * 16);
         };
-        const int64_t rps = rows_for(fill_target), least = rows_for(most_items);
-        most_splits = (int)((nl + least - 1) / least);
+        const int64_t rps = rows_for(total, fill_target);
+        // a larger rows_total takes longer splits, except past the line above
+        if (fill_target < most_items) {
+            const int64_t least = rows_for((int64_t)cu * 704, most_items);
+            most_splits = (int)((nl + least - 1) / least);
+        }
         p->lat.rows_per_split = (int)rps;
         p->lat.splits = (int)((nl + rps - 1) / rps);
         p->lat.nwg = wave_item_groups((int)B, p->lat.splits, p->lat.tiles);
@@ -2955,14 +2962,12 @@ int plan_latent(const slimkv_latent_decode_args* a, LatentPlan* p, const PagedRo
     const size_t rr = (size_t)B * Hq * Lq * p->raw.splits;
     p->rml_off = off; off = align256(off + rr * 8);
     p->racc_off = off; off = align256(off + rr * D * 4);
-    const size_t lr = (size_t)B * Hq * Lq * p->lat.splits;
-    p->lml_off = off; off = align256(off + lr * 8);
-    p->lacc_off = off; off = align256(off + lr * (size_t)rv * 4);
+    const size_t rows = (size_t)B * Hq * Lq, partials = off;
+    p->lml_off = off; off = align256(off + rows * p->lat.splits * 8);
+    p->lacc_off = off; off = align256(off + rows * p->lat.splits * (size_t)rv * 4);
     p->total = off;
-    // A workspace asked for at the largest sizes of a run serves the smaller
-    // ones too, which may take more splits.
-    const size_t more = (size_t)B * Hq * Lq * std::max(0, most_splits - p->lat.splits);
-    p->bound = off + (more ? align256(more * 8) + align256(more * (size_t)rv * 4) : 0);
+    const size_t most = rows * std::max(most_splits, p->lat.splits);
+    p->bound = align256(partials + most * 8) + align256(most * (size_t)rv * 4);
     return SLIMKV_OK;
 }
 

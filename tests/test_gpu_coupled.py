@@ -177,18 +177,39 @@ def test_two_segments_equal_joined_rows(device, first):
 
 
 # rows either side of a whole number of tiles a split, with few raw workgroups
-# (the splits leave them CUs) and with many (they do not)
-@pytest.mark.parametrize('B,raw,n', [(1, 70, 251 * 64), (1, 70, 251 * 64 + 1), (1, 70, 256 * 64 + 1), (9, 1000, 1793)])
+# (three at 70 rows: the splits leave them CUs, 253 of 256) and with many (they
+# do not)
+@pytest.mark.parametrize('B,raw,n', [(1, 70, 253 * 64), (1, 70, 253 * 64 + 1), (1, 70, 256 * 64 + 1), (9, 1000, 1793)])
 def test_split_counts(device, B, raw, n):
     check(layer(device, B, 8, 8, n, raw, 64, 64), f'{n} beacons')
 
 
+@pytest.mark.parametrize('splits', [1, 7, 66, 256])
+def test_given_splits(device, splits):
+    """4200 rows are 66 tiles: seven splits of ten tiles, 66 of one."""
+    check(layer(device, 1, 32, 8, 4200, 20, 64, 200), f'{splits} splits', lat_splits=splits)
+
+
 def test_workspace_of_more_beacons_serves_fewer(device):
-    """252 tiles of 64 rows take 126 splits, 251 tiles 251."""
-    from slimkv_amd import kernels
-    few, many = (kernels.latent_decode_workspace_bytes(*layer(device, 1, 8, 8, n * 64, 5, 64, 64)[0])
-                 for n in (251, 252))
-    assert few <= many
+    """One raw workgroup leaves all CUs but one: as many tiles of 64 rows take
+    a split each, one tile more half as many splits, and its workspace still
+    holds the partials of the smaller call."""
+    import ctypes
+    from slimkv_amd import _lib, kernels
+    cu = torch.cuda.get_device_properties(device).multi_processor_count
+    few, many = (layer(device, 1, 8, 8, tiles * 64, 5, 64, 64) for tiles in (cu - 1, cu))
+
+    def query(case, lat_splits=0):
+        return kernels.latent_decode_workspace_bytes(*case[0], lat_splits=lat_splits)
+    assert query(few) == query(few, lat_splits=cu - 1) > query(many, lat_splits=cu // 2)
+    size = query(many)
+    args, kw, out, lse, atol = few
+    a, got, got_lse, keep = kernels._latent_args(
+        *args, None, None, False, False, kw['q_positions'], kw['cos'], kw['sin'], None, None, 0, 0, None, None)
+    workspace = torch.empty(size, dtype=torch.uint8, device=device)
+    _lib.check(_lib.lib().slimkv_latent_decode(ctypes.byref(a), workspace.data_ptr(), size, _lib.stream_handle(device)))
+    assert_close(to_np(got), out.cpu().numpy(), what='workspace of more beacons')
+    assert_lse_close(to_np(got_lse), lse.cpu().numpy(), atol=atol, what='workspace of more beacons')
 
 
 def test_strided_and_shared_rows(device):

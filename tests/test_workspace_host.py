@@ -1,0 +1,49 @@
+"""Workspace queries (no GPU needed: nothing here launches a kernel): a size
+asked for once serves the calls that the header says it serves."""
+import ctypes
+
+import pytest
+
+
+def latent_args(batch, heads, beacons, rank_k, rank_v, *, queries=1, kv_heads=8, raw=133, raw_splits=0, lat_splits=0,
+                per_head=False):
+    from slimkv_amd import _lib
+    a = _lib.LatentDecodeArgs()
+    for name in ('q', 'raw_k', 'raw_v', 'lat_k', 'lat_v', 'up_k', 'up_v', 'out'):
+        setattr(a, name, 1 << 20)           # any aligned address: a query reads no data
+    a.batch, a.queries, a.heads, a.kv_heads, a.head_dim = batch, queries, heads, kv_heads, 128
+    a.raw_keys, a.lat_keys, a.rank_k, a.rank_v, a.scale = raw, beacons, rank_k, rank_v, 128 ** -0.5
+    a.raw_splits, a.lat_splits, a.block_diagonal = raw_splits, lat_splits, int(per_head)
+    return a
+
+
+def latent_workspace(*args, **kw):
+    from slimkv_amd import _lib
+    return _lib.lib().slimkv_latent_decode_workspace(ctypes.byref(latent_args(*args, **kw)))
+
+
+@pytest.mark.parametrize('batch,heads,queries,rank', [(1, 8, 1, 64), (16, 8, 1, 64), (16, 8, 1, 128), (64, 8, 1, 256),
+                                                      (1, 32, 1, 256), (8, 32, 1, 256), (3, 40, 2, 320),
+                                                      (300, 32, 1, 128)])
+def test_fewer_beacons_fit_the_workspace_of_more(batch, heads, queries, rank):
+    """Bases without blocks, automatic splits."""
+    sizes = [latent_workspace(batch, heads, n, rank, rank, queries=queries)
+             for n in sorted({*range(1, 20000, 331), *(64 * t for t in range(250, 260)), 16384, 16385})]
+    assert sizes[0] > 0 and sizes == sorted(sizes)
+
+
+@pytest.mark.parametrize('rank', [128, 256])
+@pytest.mark.parametrize('sequences', [8, 55, 56])
+def test_a_larger_row_total_fits_the_workspace_of_a_smaller(sequences, rank):
+    from slimkv_amd import _lib
+    sizes = []
+    for total in [65543, *range(704 * 256 - 900, 704 * 256 + 1200, 300), 704 * 256 - 1, 704 * 256, 1 << 18, 1 << 19]:
+        a = _lib.PagedLatentDecodeArgs()
+        a.base = latent_args(sequences, 32, 65536, rank, rank, per_head=True)
+        a.base.lat_lengths = a.pages = a.table = 1 << 20
+        a.slots, a.sink_elements, a.page_stride, a.num_pages = 4, 0, 8 * rank, 1 << 20
+        a.t_cols = a.t_sb = 1 << 14
+        a.rows_total = total
+        sizes.append((total, _lib.lib().slimkv_paged_latent_decode_workspace(ctypes.byref(a))))
+    sizes = [size for _, size in sorted(sizes)]
+    assert sizes[-1] > 0 and sizes == sorted(sizes, reverse=True)

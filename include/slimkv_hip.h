@@ -178,7 +178,7 @@ int slimkv_latent_decode_stages(const slimkv_latent_decode_args* a, int stages, 
  * overlap on a GPU (other streams, other threads) race and must be ordered by
  * the caller.  The array needs no clearing between calls.  Results equal
  * slimkv_latent_decode's. */
-#define SLIMKV_NOALLOC_SCRATCH_BYTES (32u << 20)
+#define SLIMKV_NOALLOC_SCRATCH_BYTES (64u << 20)
 int slimkv_latent_decode_noalloc(const slimkv_latent_decode_args* a, void* stream);
 
 /* ------------------------------------------------------------------------

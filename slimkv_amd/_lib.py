@@ -282,7 +282,7 @@ SIGNATURES = {
 ABI_VERSION = 15
 
 STAGE_PROLOGUE, STAGE_ATTEND, STAGE_COMBINE, STAGE_ALL = 1, 2, 4, 7
-NOALLOC_SCRATCH_BYTES = 32 << 20
+NOALLOC_SCRATCH_BYTES = 64 << 20
 STATUS_BAD_PAGE = 1
 STATUS_BAD_SLOT = 2
 

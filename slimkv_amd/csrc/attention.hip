@@ -2923,10 +2923,9 @@ int plan_latent(const slimkv_latent_decode_args* a, LatentPlan* p, const PagedRo
             most_splits = std::max(most_splits, std::min({std::max(1, cu / ((int)B * p->groups)), tiles64, kMaxSplits}));
             const int free_cus = 4 * p->raw.nwg <= cu ? cu - p->raw.nwg : cu;
             splits = (int)std::max<int64_t>(1, free_cus / ((int64_t)B * p->groups));
-            const int longest = (tiles64 + splits - 1) / splits;
-            splits = (tiles64 + longest - 1) / longest;
         }
-        splits = std::min({splits, tiles64, kMaxSplits});
+        const int longest = (tiles64 + std::min(splits, kMaxSplits) - 1) / std::min(splits, kMaxSplits);
+        splits = (tiles64 + longest - 1) / longest;
         p->lat.splits = splits;
         p->lat.rows_per_split = 0;
         p->lat.nwg = (int)B * splits * p->groups;
@@ -3187,8 +3186,12 @@ extern "C" int slimkv_latent_decode_stages(const slimkv_latent_decode_args* a, i
 // ---------------------------------------------------------------------------
 
 // One copy per GPU, allocated when the library's code object is loaded on that
-// GPU and held until the process ends.  In host code `scratch` names a
-// host-side stand-in: its device address comes from hipGetSymbolAddress.
+// GPU and held until the process ends.  Its size: a coupled plan's partials are
+// at most 20,480 rows of 384 columns (a workgroup a CU, 80 query rows each),
+// 30.2 MiB; the other half holds the raw partials and the query operands of
+// every call that fitted 32 MiB with the split kernel's fewer splits.  In host
+// code `scratch` names a host-side stand-in: its device address comes from
+// hipGetSymbolAddress.
 static __device__ __align__(256) unsigned char scratch[SLIMKV_NOALLOC_SCRATCH_BYTES];
 
 namespace {
@@ -3221,23 +3224,15 @@ extern "C" int slimkv_latent_decode_noalloc(const slimkv_latent_decode_args* a, 
     LatentPlan p{};
     int rc = plan_latent(a, &p);
     if (rc != SLIMKV_OK) return rc;
-    // Coupled bases plan a workgroup a CU, up to 80 query rows each: fewer
-    // splits where their partials would not fit.
-    slimkv_latent_decode_args fit = *a;
-    while (p.coupled && p.total > (size_t)SLIMKV_NOALLOC_SCRATCH_BYTES && p.lat.splits > 1) {
-        fit.lat_splits = p.lat.splits / 2;
-        rc = plan_latent(&fit, &p);
-        if (rc != SLIMKV_OK) return rc;
-    }
-    if (p.total > (size_t)SLIMKV_NOALLOC_SCRATCH_BYTES)
-        return fail(SLIMKV_EWORKSPACE, "slimkv_latent_decode_noalloc: this call needs " + std::to_string(p.total) +
+    if (p.bound > (size_t)SLIMKV_NOALLOC_SCRATCH_BYTES)
+        return fail(SLIMKV_EWORKSPACE, "slimkv_latent_decode_noalloc: this call needs " + std::to_string(p.bound) +
                                            " bytes of workspace, more than the " +
                                            std::to_string((size_t)SLIMKV_NOALLOC_SCRATCH_BYTES) +
                                            "-byte device scratch; use slimkv_latent_decode with a caller workspace");
     void* ws = nullptr;
     rc = scratch_address(&ws);
     if (rc != SLIMKV_OK) return rc;
-    return latent_decode_run(&fit, nullptr, ws, (size_t)SLIMKV_NOALLOC_SCRATCH_BYTES, stream);
+    return latent_decode_run(a, nullptr, ws, (size_t)SLIMKV_NOALLOC_SCRATCH_BYTES, stream);
 }
 
 extern "C" size_t slimkv_paged_latent_decode_workspace(const slimkv_paged_latent_decode_args* a) {

@@ -47,3 +47,29 @@ def test_a_larger_row_total_fits_the_workspace_of_a_smaller(sequences, rank):
         sizes.append((total, _lib.lib().slimkv_paged_latent_decode_workspace(ctypes.byref(a))))
     sizes = [size for _, size in sorted(sizes)]
     assert sizes[-1] > 0 and sizes == sorted(sizes, reverse=True)
+
+
+def test_device_scratch_constant_matches_the_header():
+    import re
+    from pathlib import Path
+    from slimkv_amd import _lib
+    header = (Path(__file__).resolve().parents[1] / 'include' / 'slimkv_hip.h').read_text()
+    mib = int(re.search(r'SLIMKV_NOALLOC_SCRATCH_BYTES \((\d+)u << 20\)', header).group(1))
+    assert _lib.NOALLOC_SCRATCH_BYTES == mib << 20
+
+
+@pytest.mark.parametrize('batch,heads,queries', [(1, 40, 2), (3, 40, 2), (16, 40, 2), (51, 40, 2), (2, 96, 1),
+                                                 (64, 32, 1), (128, 32, 2), (256, 8, 1)])
+@pytest.mark.parametrize('rank_v', [256, 384])
+def test_the_device_scratch_holds_coupled_partials(batch, heads, queries, rank_v):
+    """The allocation-free call has a fixed scratch: with few raw rows it takes
+    every coupled plan up to 256 sequences, whatever its beacons, and a given
+    split count takes no more than it says."""
+    from slimkv_amd import _lib
+    for beacons in (64, 1000, 4096, 16384, 100000):
+        assert 0 < latent_workspace(batch, heads, beacons, 384, rank_v, queries=queries, raw=64) <= _lib.NOALLOC_SCRATCH_BYTES
+    for beacons in (130, 1000, 4200):
+        given = [latent_workspace(batch, heads, beacons, 384, rank_v, queries=queries, lat_splits=n) for n in range(1, 40)]
+        rows = batch * heads * queries
+        for n, size in enumerate(given, 1):
+            assert size <= given[0] + (n - 1) * rows * (4 * rank_v + 8) + 512

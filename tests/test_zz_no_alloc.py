@@ -55,7 +55,7 @@ def test_two_calls_in_a_row_match_the_workspace_entry_point(device, cases):
 def test_call_larger_than_the_scratch_is_refused(device):
     """64 sequences with 1024 raw rows read in 64 raw splits (asked for) need
     512 fp32 partial bytes per split and query head: about 68 MB of workspace,
-    over the 32 MiB scratch."""
+    over the 64 MiB scratch."""
     from slimkv_amd import _lib, kernels
     case = latent_case(batch=2, context=600, tail=20, seed=73, device=device)
     B, Nr = 64, 1024

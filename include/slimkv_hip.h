@@ -48,8 +48,9 @@ int slimkv_abi_version(void);
 
 /* Stages of a decode call, for the *_stages entry points (bit mask).  A
  * decode runs three kernels that hand over through the caller's workspace:
- *   SLIMKV_STAGE_PROLOGUE  query RoPE (and, for the latent decode, the query
- *                          absorption into U_K and the K-bias LSE shift);
+ *   SLIMKV_STAGE_PROLOGUE  the latent decode's query RoPE, its absorption into
+ *                          U_K and the K-bias LSE shift (the reconstruction
+ *                          decode rotates its queries at the attend stage);
  *   SLIMKV_STAGE_ATTEND    the split-K attention: per-split partials;
  *   SLIMKV_STAGE_COMBINE   the LSE merge of the partials, the V lift, out/lse.
  * A *_stages call runs the selected stages in that order.  Calls with the
@@ -338,10 +339,9 @@ int slimkv_prepare_rope_pairs(const float* cos, const float* sin, int64_t rows, 
 size_t slimkv_recon_decode_workspace(const slimkv_recon_decode_args* a);
 int slimkv_recon_decode(const slimkv_recon_decode_args* a, void* workspace, size_t workspace_bytes, void* stream);
 /* slimkv_recon_decode restricted to `stages` (SLIMKV_STAGE_*): the prologue
- * rotates the query, except on the fused route (K rebuilt per tile inside the
- * split kernel), whose split kernel rotates its query rows itself and whose
- * prologue stage does nothing; the attend stage rebuilds what the route
- * rebuilds and runs the split kernel. */
+ * stage does nothing; the attend stage rebuilds what the route rebuilds and
+ * runs the split kernel, which rotates the query rows where it reads them, so
+ * q, q_positions and the tables stay as they are until it has run. */
 int slimkv_recon_decode_stages(const slimkv_recon_decode_args* a, int stages, void* workspace,
                                size_t workspace_bytes, void* stream);
 

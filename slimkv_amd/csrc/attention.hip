@@ -1053,7 +1053,6 @@ namespace slimkv {
 // tables whose rows repeat their first half (cos[d] = cos[d + 64]), which the
 // caller checks once per table.
 struct ReconSeg {
-    const uint16_t* q; int64_t q_sb, q_sl, q_sh;        // rotated queries [B, Lq, Hq, 128]
     const uint16_t* lk; int64_t lk_sb, lk_sn;           // latent K rows, head h at [h*rk, (h+1)*rk)
     const uint16_t* lv; int64_t lv_sb, lv_sn;           // latent V rows, head h at [h*rv, (h+1)*rv)
     const uint16_t* w; const uint16_t* bias; int64_t w_ld;   // U_K [Hkv*128, Rk] (nn.Linear), bias or null
@@ -1063,7 +1062,7 @@ struct ReconSeg {
     int n, hk, g, causal;
     int splits, rows_per_split, nwg;
     float* part_ml; float* part_acc;                    // partials, rv wide
-    QRope qr;                                           // q null: q above holds rotated rows
+    QRope qr;                                           // the queries as given
 };
 
 // One 16-key tile of latent rows in registers, with the key position of the
@@ -1193,52 +1192,42 @@ __device__ __forceinline__ void recon_segment(const ReconSeg& sg, int w, int Lq,
                               : v4f{0.f, 0.f, 0.f, 0.f};
     // Rotated query of the column (B operand of the scores): d = 16t + 4grp + [0, 4).
     u32x2 qop[8];
-    if (sg.qr.q) {
-        // Rotated here from the query as given, with the reference's bf16
-        // steps (as rope_operand): element 16t + 4grp + e has its rotate-half
-        // partner at t ^ 4 in the same lane.
-        const uint16_t* qrow = sg.qr.q + (int64_t)b * sg.qr.q_sb + (int64_t)lq * sg.qr.q_sl + (int64_t)j * sg.qr.q_sh +
-                               4 * grp;
-        u32x2 x[8];
+    // Rotated here from the query as given, with the reference's bf16
+    // steps (as rope_operand): element 16t + 4grp + e has its rotate-half
+    // partner at t ^ 4 in the same lane.
+    const uint16_t* qrow = sg.qr.q + (int64_t)b * sg.qr.q_sb + (int64_t)lq * sg.qr.q_sl + (int64_t)j * sg.qr.q_sh + 4 * grp;
+    u32x2 x[8];
 #pragma unroll
-        for (int tt = 0; tt < 8; ++tt) x[tt] = *reinterpret_cast<const u32x2*>(qrow + 16 * tt);
-        if (sg.qr.cos) {
-            const int64_t row = qrope_row(sg.qr, b, lq, Lq);
-            float4 cs[8], sn[8];
-#pragma unroll
-            for (int tt = 0; tt < 8; ++tt) {
-                cs[tt] = *reinterpret_cast<const float4*>(sg.qr.cos + row * 128 + 16 * tt + 4 * grp);
-                sn[tt] = *reinterpret_cast<const float4*>(sg.qr.sin + row * 128 + 16 * tt + 4 * grp);
-            }
-            float v[8][4];
-#pragma unroll
-            for (int tt = 0; tt < 8; ++tt) {
-                v[tt][0] = lo_bf16(x[tt].x); v[tt][1] = hi_bf16(x[tt].x);
-                v[tt][2] = lo_bf16(x[tt].y); v[tt][3] = hi_bf16(x[tt].y);
-            }
-#pragma unroll
-            for (int tt = 0; tt < 8; ++tt) {
-                const float cv[4] = {cs[tt].x, cs[tt].y, cs[tt].z, cs[tt].w};
-                const float sv[4] = {sn[tt].x, sn[tt].y, sn[tt].z, sn[tt].w};
-                float o[4];
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const float partner = tt < 4 ? -v[tt ^ 4][e] : v[tt ^ 4][e];
-                    o[e] = round_bf16_hw(v[tt][e] * round_bf16_hw(cv[e])) + round_bf16_hw(partner * round_bf16_hw(sv[e]));
-                }
-                x[tt] = u32x2{pack_bf16(o[0], o[1]), pack_bf16(o[2], o[3])};
-            }
-        }
-#pragma unroll
-        for (int tt = 0; tt < 8; ++tt) qop[tt] = u32x2{colv ? x[tt].x : 0u, colv ? x[tt].y : 0u};
-    } else {
-        const uint16_t* qrow = sg.q + (int64_t)b * sg.q_sb + (int64_t)lq * sg.q_sl + (int64_t)j * sg.q_sh + 4 * grp;
+    for (int tt = 0; tt < 8; ++tt) x[tt] = *reinterpret_cast<const u32x2*>(qrow + 16 * tt);
+    if (sg.qr.cos) {
+        const int64_t row = qrope_row(sg.qr, b, lq, Lq);
+        float4 cs[8], sn[8];
 #pragma unroll
         for (int tt = 0; tt < 8; ++tt) {
-            const u32x2 x = *reinterpret_cast<const u32x2*>(qrow + 16 * tt);
-            qop[tt] = u32x2{colv ? x.x : 0u, colv ? x.y : 0u};
+            cs[tt] = *reinterpret_cast<const float4*>(sg.qr.cos + row * 128 + 16 * tt + 4 * grp);
+            sn[tt] = *reinterpret_cast<const float4*>(sg.qr.sin + row * 128 + 16 * tt + 4 * grp);
+        }
+        float v[8][4];
+#pragma unroll
+        for (int tt = 0; tt < 8; ++tt) {
+            v[tt][0] = lo_bf16(x[tt].x); v[tt][1] = hi_bf16(x[tt].x);
+            v[tt][2] = lo_bf16(x[tt].y); v[tt][3] = hi_bf16(x[tt].y);
+        }
+#pragma unroll
+        for (int tt = 0; tt < 8; ++tt) {
+            const float cv[4] = {cs[tt].x, cs[tt].y, cs[tt].z, cs[tt].w};
+            const float sv[4] = {sn[tt].x, sn[tt].y, sn[tt].z, sn[tt].w};
+            float o[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float partner = tt < 4 ? -v[tt ^ 4][e] : v[tt ^ 4][e];
+                o[e] = round_bf16_hw(v[tt][e] * round_bf16_hw(cv[e])) + round_bf16_hw(partner * round_bf16_hw(sv[e]));
+            }
+            x[tt] = u32x2{pack_bf16(o[0], o[1]), pack_bf16(o[2], o[3])};
         }
     }
+#pragma unroll
+    for (int tt = 0; tt < 8; ++tt) qop[tt] = u32x2{colv ? x[tt].x : 0u, colv ? x[tt].y : 0u};
 
     ReconTile<KSR, VL> ring[kReconRing];
     u32x4 pairs[2][4];
@@ -3267,7 +3256,7 @@ struct ReconPlan {
     SegPlan raw, rec;
     int v_latent, v_width;   // V stays latent (width v_width per KV head) and is lifted in the combine
     int fused, ksr, vl;      // K rebuilt per tile inside the split kernel (recon_split_kernel<ksr, vl>)
-    size_t qrot_off, k_off, v_off, rml_off, racc_off, bml_off, bacc_off, total;
+    size_t k_off, v_off, rml_off, racc_off, bml_off, bacc_off, total;
 };
 
 // The fused route: block-diagonal bases, per-head K rank 16, 32 or 48 and V
@@ -3359,7 +3348,6 @@ int plan_recon(const slimkv_recon_decode_args* r, ReconPlan* p) {
     size_t off = 0;
     p->v_latent = (p->fused || recon_v_latent(a)) ? 1 : 0;
     p->v_width = p->v_latent ? (int)(a->block_diagonal ? a->rank_v / Hkv : a->rank_v) : (int)D;
-    p->qrot_off = off; off = align256(off + (size_t)B * Lq * Hq * D * 2);
     p->k_off = off; off = align256(off + (p->fused ? 0 : (size_t)B * nl * Hkv * D * 2));
     p->v_off = off; off = align256(off + (p->v_latent ? 0 : (size_t)B * nl * Hkv * D * 2));
     const size_t rr = (size_t)B * Hq * Lq * p->raw.splits;
@@ -3373,9 +3361,8 @@ int plan_recon(const slimkv_recon_decode_args* r, ReconPlan* p) {
 }
 
 // Raw rows and rebuilt-per-tile beacon rows in one launch, then the combine
-// with the latent V lift.  q_rot already holds the rotated queries.
-int recon_fused_run(const slimkv_recon_decode_args* r, const ReconPlan& p, char* ws, uint16_t* q_rot, hipStream_t st,
-                    int stages) {
+// with the latent V lift.
+int recon_fused_run(const slimkv_recon_decode_args* r, const ReconPlan& p, char* ws, hipStream_t st, int stages) {
     const slimkv_latent_decode_args* a = &r->base;
     const int B = (int)a->batch, Lq = (int)a->queries, Hq = (int)a->heads, Hkv = (int)a->kv_heads, D = (int)a->head_dim;
     const int g = Hq / Hkv;
@@ -3384,7 +3371,6 @@ int recon_fused_run(const slimkv_recon_decode_args* r, const ReconPlan& p, char*
     prm.scale_log2 = (float)(a->scale * 1.4426950408889634);
     prm.nseg = 1;
     Seg& rs = prm.seg[0];
-    rs.q = q_rot; rs.q_sb = (int64_t)Lq * Hq * D; rs.q_sl = (int64_t)Hq * D; rs.q_sh = D;
     rs.k = static_cast<const uint16_t*>(a->raw_k); rs.k_sb = a->rk_sb; rs.k_sn = a->rk_sn; rs.k_sh = a->rk_sh;
     rs.v = static_cast<const uint16_t*>(a->raw_v); rs.v_sb = a->rv_sb; rs.v_sn = a->rv_sn; rs.v_sh = a->rv_sh;
     rs.seqlens = a->raw_lengths; rs.n = (int)a->raw_keys;
@@ -3399,7 +3385,6 @@ int recon_fused_run(const slimkv_recon_decode_args* r, const ReconPlan& p, char*
     qr.cos = a->cos; qr.sin = a->sin; qr.rope_rows = a->rope_rows;
 
     ReconSeg bs{};
-    bs.q = q_rot; bs.q_sb = rs.q_sb; bs.q_sl = rs.q_sl; bs.q_sh = rs.q_sh;
     bs.qr = qr;
     bs.lk = static_cast<const uint16_t*>(a->lat_k); bs.lk_sb = a->lk_sb; bs.lk_sn = a->lk_sn;
     bs.lv = static_cast<const uint16_t*>(a->lat_v); bs.lv_sb = a->lv_sb; bs.lv_sn = a->lv_sn;
@@ -3470,13 +3455,12 @@ int recon_decode_run(const slimkv_recon_decode_args* r, void* workspace, size_t 
     const int B = (int)a->batch, Lq = (int)a->queries, Hq = (int)a->heads, Hkv = (int)a->kv_heads, D = (int)a->head_dim;
     const int g = Hq / Hkv;
     const bool has_lat = a->lat_keys > 0;
-    uint16_t* q_rot = reinterpret_cast<uint16_t*>(ws + p.qrot_off);
     uint16_t* kbuf = reinterpret_cast<uint16_t*>(ws + p.k_off);
     uint16_t* vbuf = reinterpret_cast<uint16_t*>(ws + p.v_off);
 
     // 1. The split kernels rotate the queries where they read them: no prologue
     // launch (the prologue stage does nothing).
-    if (p.fused) return recon_fused_run(r, p, ws, q_rot, st, stages);
+    if (p.fused) return recon_fused_run(r, p, ws, st, stages);
 
     // 2. rebuild beacon K (optionally RoPE'd) and, unless it stays latent, V: [B, Nl, Hkv, D]
     if (has_lat && (stages & SLIMKV_STAGE_ATTEND)) {
@@ -3509,7 +3493,6 @@ int recon_decode_run(const slimkv_recon_decode_args* r, void* workspace, size_t 
     prm.qrope = QRope{static_cast<const uint16_t*>(a->q), a->q_sb, a->q_sl, a->q_sh, a->q_positions, a->pos_sb, a->cos,
                       a->sin, a->rope_rows};
     Seg& rs = prm.seg[has_lat ? 1 : 0];
-    rs.q = q_rot; rs.q_sb = (int64_t)Lq * Hq * D; rs.q_sl = (int64_t)Hq * D; rs.q_sh = D;
     rs.k = static_cast<const uint16_t*>(a->raw_k); rs.k_sb = a->rk_sb; rs.k_sn = a->rk_sn; rs.k_sh = a->rk_sh;
     rs.v = static_cast<const uint16_t*>(a->raw_v); rs.v_sb = a->rv_sb; rs.v_sn = a->rv_sn; rs.v_sh = a->rv_sh;
     rs.seqlens = a->raw_lengths; rs.n = (int)a->raw_keys;

@@ -28,7 +28,7 @@ pytestmark = pytest.mark.gpu
 def test_reconstruct_matches_oracle_gemm(device, bd, rank, bias, B, n):
     """Per-head widths up to 64 take the streaming kernel (several 16-row tiles per
     wavefront once B * Hkv * rows / 64 exceeds its workgroup budget, ragged last
-    tile); wider contractions the per-tile kernel."""
+    tile), 128 and wider the one that keeps W in registers."""
     from slimkv_amd import kernels
     gen = torch.Generator(device=device).manual_seed(rank + n)
     Hkv, D = 8, 128

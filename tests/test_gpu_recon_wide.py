@@ -8,7 +8,7 @@ import torch
 from oracle import attention as oa
 from oracle import rope as orope
 from slimkv_amd.workloads import rope_tables
-from tests.helpers import neighbour_of_exact, to_np
+from tests.helpers import assert_close, neighbour_of_exact, to_np
 
 pytestmark = pytest.mark.gpu
 
@@ -117,3 +117,54 @@ def test_forward_mode_reaches_the_rows_around_a_history(device):
         got, tangent = forward_ad.unpack_dual(cache.materialize(attention, forward_ad.make_dual(current, dcurrent)))
     assert torch.equal(got, plain)
     assert torch.equal(tangent, torch.cat([dsink, torch.zeros_like(tangent[:, :, 4:24]), dcurrent], 2))
+
+
+@pytest.mark.parametrize('repeats', [True, False])
+@pytest.mark.parametrize('R,B,n', [(256, 1, 33), (256, 2, 2100), (128, 2, 700), (384, 1, 17), (512, 1, 40), (512, 2, 1100)])
+def test_decode_over_rebuilt_rotated_keys(device, R, B, n, repeats):
+    """The reconstruction decode on coupled bases with beacon positions: RoPE
+    from prepared pairs (rows that repeat their first half and rows that do
+    not) and from the tables give the same bits; against float64 attention over
+    the rows that reconstruct writes; stage by stage as in one call, with a
+    prologue stage that leaves the workspace alone."""
+    import ctypes
+    from slimkv_amd import _lib, kernels
+    gen = torch.Generator(device=device).manual_seed(R + n)
+
+    def rnd(*shape, std=1.0):
+        return (torch.randn(*shape, generator=gen, device=device) * std).to(torch.bfloat16)
+    Hq, raw = 32, 21
+    q, raw_k, raw_v = rnd(B, 1, Hq, D), rnd(B, raw, HKV, D), rnd(B, raw, HKV, D)
+    lk, lv = rnd(B, n, R), rnd(B, n, R)
+    uk, uv = rnd(HKV * D, R, std=R ** -0.5), rnd(HKV * D, R, std=R ** -0.5)
+    bk, bv = rnd(HKV * D, std=0.1), rnd(HKV * D, std=0.1)
+    cos, sin = rope_tables(4000, D, 500000.0, device)
+    if not repeats:
+        cos, sin = (torch.cat([t[:, :64], t[:, 64:].roll(7, 0)], 1).contiguous() for t in (cos, sin))
+    assert bool(kernels.prepare_rope_pairs(cos, sin)[1]) == repeats
+    pos = torch.full((B, 1), 3333, dtype=torch.int64, device=device)
+    beacons = torch.randint(0, 4000, (B, n), generator=gen, device=device)
+    kw = dict(beacon_positions=beacons, up_k_bias=bk, up_v_bias=bv, q_positions=pos, cos=cos, sin=sin)
+    out, lse = kernels.recon_decode(q, raw_k, raw_v, lk, lv, uk, uv, D ** -0.5, **kw)
+
+    base, plain, plain_lse, keep = kernels._latent_args(
+        q, raw_k, raw_v, lk, lv, uk, uv, D ** -0.5, bk, bv, False, False, pos, cos, sin, None, None, 0, 0, None, None,
+        prepared_bases=False)
+    a = _lib.ReconDecodeArgs(base, beacons.data_ptr(), n, None, 0, 0)
+    size = _lib.lib().slimkv_recon_decode_workspace(ctypes.byref(a))
+    ws = torch.full((size,), 7, dtype=torch.uint8, device=device)
+    for stage in (_lib.STAGE_PROLOGUE, _lib.STAGE_ATTEND, _lib.STAGE_COMBINE):
+        _lib.check(_lib.lib().slimkv_recon_decode_stages(ctypes.byref(a), stage, ws.data_ptr(), size,
+                                                         _lib.stream_handle(device)))
+        assert stage != _lib.STAGE_PROLOGUE or bool((ws == 7).all())
+    assert torch.equal(out, plain) and torch.equal(lse, plain_lse)
+
+    key = kernels.reconstruct(lk, uk, bk, kv_heads=HKV, positions=beacons, cos=cos, sin=sin).double()
+    value = kernels.reconstruct(lv, uv, bv, kv_heads=HKV).double()
+    c, s = cos.to(torch.bfloat16).double()[3333], sin.to(torch.bfloat16).double()[3333]
+    x = q[:, 0].double()
+    x = (x * c + torch.cat([-x[..., 64:], x[..., :64]], -1) * s).view(B, HKV, Hq // HKV, D)
+    key, value = (torch.cat([t, u.double()], 1).transpose(1, 2) for t, u in ((key, raw_k), (value, raw_v)))
+    sc = x @ key.transpose(-1, -2).contiguous() * D ** -0.5
+    assert_close(to_np(out[:, 0]), (torch.softmax(sc, -1) @ value.contiguous()).reshape(B, Hq, D).cpu().numpy(),
+                 what=f'width {R}')

@@ -2290,78 +2290,104 @@ prologue_mfma_kernel(PrologueParams pp) {
 }
 
 // MFMA prologue over U_K as given (coupled bases, and per-head ones without a
-// prepared transpose): a workgroup per (b, KV head, 64 latent columns), a wave
-// per 16 of them, q_lat^T[k][p] = U_K[:, k]^T . q_rot[p][:].  The head's 128 x
-// 64 block of U_K goes through LDS, where transposing reads make the A operand
-// (rows 32 bytes past a multiple of 128, so four rows meet distinct banks);
-// every wave rotates the query rows itself.  One memory round trip and the
-// launch bound it; prologue_kernel's threads walk the head's rows eight at a
-// time (four query rows and width 256: 8.4 -> 4.2 us, ten and 320: 20 -> 5.4)
-// and stay for query rows, U_K or biases off a 16-byte boundary.
+// prepared transpose): a workgroup per (b, KV head) and every `groups`-th block
+// of 64 latent columns, a wave per 16 of them, q_lat^T[k][p] = U_K[:, k]^T .
+// q_rot[p][:].  The head's 128 x 64 block of U_K goes through LDS, where
+// transposing reads make the A operand (rows 32 bytes past a multiple of 128, so
+// four rows meet distinct banks); every wave with columns rotates the query rows
+// itself.  One memory round trip and the launch bound it.
+template <bool SEVERAL>      // blocks a workgroup
 __global__ void __launch_bounds__(256)
-prologue_wide_kernel(PrologueParams pp) {
+prologue_wide_kernel(PrologueParams pp, int groups) {
     constexpr int D = 128, STRIDE = 160;
     __shared__ __attribute__((aligned(16))) char lds[D * STRIDE];
-    const int chunks = (pp.wq + 63) / 64;
-    const int k0 = 64 * (blockIdx.x % chunks);
-    const int h = blockIdx.x / chunks % pp.Hkv;
-    const int b = blockIdx.x / chunks / pp.Hkv;
+    const int first_k = 64 * (blockIdx.x % groups);
+    const int h = blockIdx.x / groups % pp.Hkv;
+    const int b = blockIdx.x / groups / pp.Hkv;
     const int g = pp.Hq / pp.Hkv;
     const int rows = g * pp.Lq;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, col = lane & 15, grp = lane >> 4;
+    const int tid = threadIdx.x, lane = tid & 63, col = lane & 15, grp = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const bool valid = col < rows;
     const int p = valid ? col : 0;
     const int l = p % pp.Lq, j = h * g + p / pp.Lq;
 
-    // rows tid / 8 + 32 i of the block, 16-byte piece tid % 8 (pieces past the
-    // width repeat the first one; their columns are not stored)
-    const int kp = k0 + 8 * (tid % 8) < pp.wq ? k0 + 8 * (tid % 8) : 0;
-    const uint16_t* ub = pp.up_k + ((int64_t)h * D + tid / 8) * pp.Rk + (pp.blockdiag ? h * pp.wq : 0) + kp;
+    // rows tid / 8 + 32 i of a block, 16-byte piece tid % 8 (pieces past the
+    // width repeat the row's first one; their columns are not stored)
+    const uint16_t* ub = pp.up_k + ((int64_t)h * D + tid / 8) * pp.Rk + (pp.blockdiag ? h * pp.wq : 0);
     u32x4 u[4];
+    auto fetch = [&](int k0) {
+        const int kp = k0 + 8 * (tid % 8) < pp.wq ? k0 + 8 * (tid % 8) : 0;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) u[i] = *reinterpret_cast<const u32x4*>(ub + (int64_t)32 * i * pp.Rk);
-    u32x4 qr[4];
-    const uint16_t* qrow = pp.q + (int64_t)b * pp.q_sb + (int64_t)l * pp.q_sl + (int64_t)j * pp.q_sh + 8 * grp;
+        for (int i = 0; i < 4; ++i) u[i] = *reinterpret_cast<const u32x4*>(ub + (int64_t)32 * i * pp.Rk + kp);
+    };
+    auto stage = [&] {
 #pragma unroll
-    for (int c = 0; c < 4; ++c) qr[c] = *reinterpret_cast<const u32x4*>(qrow + 32 * c);
-    RopeRow rr;
-    if (pp.cos) {
-        const int64_t pos = query_rope_row(pp, b, l);
-        load_rope_row(rr, pp.cos + pos * D, pp.sin + pos * D, grp);
-    }
-    const bool first = k0 == 0 && wave == 0;            // writes the rotated rows and the shift
-    u32x4 kb[4];
-    if (pp.shift && first) {
-        const uint16_t* bk = pp.up_k_bias + (int64_t)h * D + 8 * grp;
-#pragma unroll
-        for (int c = 0; c < 4; ++c) kb[c] = *reinterpret_cast<const u32x4*>(bk + 32 * c);
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) *reinterpret_cast<u32x4*>(lds + (tid / 8 + 32 * i) * STRIDE + 16 * (tid % 8)) = u[i];
-#pragma unroll
-    for (int c = 0; c < 4; ++c) qr[c] = zero_unless(valid, qr[c]);
-    if (pp.cos) rope_operand(qr, rr);
+        for (int i = 0; i < 4; ++i) *reinterpret_cast<u32x4*>(lds + (tid / 8 + 32 * i) * STRIDE + 16 * (tid % 8)) = u[i];
+    };
+    fetch(first_k);
+    const bool own = first_k + 16 * wave < pp.wq;           // wave-uniform: the wave has columns
+    const bool first = first_k == 0 && wave == 0;           // writes the rotated rows and the shift
+    u32x4 qr[4] = {};
     const int64_t prow = ((int64_t)b * pp.Lq + l) * pp.Hq + j;
-    if (first && valid) {
+    if (own) {
+        const uint16_t* qrow = pp.q + (int64_t)b * pp.q_sb + (int64_t)l * pp.q_sl + (int64_t)j * pp.q_sh + 8 * grp;
 #pragma unroll
-        for (int c = 0; c < 4; ++c) *reinterpret_cast<u32x4*>(pp.q_rot + prow * D + 32 * c + 8 * grp) = qr[c];
-    }
-    __syncthreads();
-    v4f t4 = {0.f, 0.f, 0.f, 0.f};
+        for (int c = 0; c < 4; ++c) qr[c] = *reinterpret_cast<const u32x4*>(qrow + 32 * c);
+        RopeRow rr;
+        if (pp.cos) {
+            const int64_t pos = query_rope_row(pp, b, l);
+            load_rope_row(rr, pp.cos + pos * D, pp.sin + pos * D, grp);
+        }
+        u32x4 kb[4];
+        if (pp.shift && first) {
+            const uint16_t* bk = pp.up_k_bias + (int64_t)h * D + 8 * grp;
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-        const char* src = lds + (32 * c + 8 * grp + (col >> 2)) * STRIDE + 2 * (16 * wave + 4 * (col & 3));
-        const u32x2 lo = __builtin_bit_cast(u32x2, read_transposed(src));
-        const u32x2 hi = __builtin_bit_cast(u32x2, read_transposed(src + 4 * STRIDE));
-        t4 = mfma32(u32x4{lo.x, lo.y, hi.x, hi.y}, qr[c], t4);
+            for (int c = 0; c < 4; ++c) kb[c] = *reinterpret_cast<const u32x4*>(bk + 32 * c);
+        }
+        stage();
+#pragma unroll
+        for (int c = 0; c < 4; ++c) qr[c] = zero_unless(valid, qr[c]);
+        if (pp.cos) rope_operand(qr, rr);
+        if (first && valid) {
+#pragma unroll
+            for (int c = 0; c < 4; ++c) *reinterpret_cast<u32x4*>(pp.q_rot + prow * D + 32 * c + 8 * grp) = qr[c];
+        }
+        if (pp.shift && first) {
+            const float dot = kbias_dot(qr, kb);
+            if (valid && grp == 0) pp.shift[(int64_t)b * pp.Hq * pp.Lq + j * pp.Lq + l] = dot * pp.scale;
+        }
     }
-    const int k = k0 + 16 * wave + 4 * grp;
-    if (valid && k < pp.wq)
-        *reinterpret_cast<u32x2*>(pp.q_lat + prow * pp.wq + k) = u32x2{pack_bf16(t4[0], t4[1]), pack_bf16(t4[2], t4[3])};
-    if (pp.shift && first) {
-        const float dot = kbias_dot(qr, kb);
-        if (valid && grp == 0) pp.shift[(int64_t)b * pp.Hq * pp.Lq + j * pp.Lq + l] = dot * pp.scale;
+    if (!own) stage();
+    for (int k0 = first_k;; k0 += 64 * groups) {
+        __syncthreads();
+        const bool more = SEVERAL && k0 + 64 * groups < pp.wq;
+        if (more) fetch(k0 + 64 * groups);
+        v4f t4 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const char* src = lds + (32 * c + 8 * grp + (col >> 2)) * STRIDE + 2 * (16 * wave + 4 * (col & 3));
+            const u32x2 lo = __builtin_bit_cast(u32x2, read_transposed(src));
+            const u32x2 hi = __builtin_bit_cast(u32x2, read_transposed(src + 4 * STRIDE));
+            t4 = mfma32(u32x4{lo.x, lo.y, hi.x, hi.y}, qr[c], t4);
+        }
+        const int k = k0 + 16 * wave + 4 * grp;
+        if (valid && k < pp.wq)
+            *reinterpret_cast<u32x2*>(pp.q_lat + prow * pp.wq + k) = u32x2{pack_bf16(t4[0], t4[1]), pack_bf16(t4[2], t4[3])};
+        if (!more) break;
+        __syncthreads();                                    // every wave is past its reads of this block
+        stage();
     }
+}
+
+// Workgroups a (sequence, KV head) of the kernel above: a block of columns each
+// while two a CU hold them all, else several blocks each, so that the query
+// rows are read and rotated less often (32 heads, width 384, 64 sequences: 7.8
+// us, 15.9 with a workgroup a block; 256 sequences 20.7 / 53.7; 16 sequences 5.5
+// / 6.0; one to eight sequences 4.2-4.4, all widths).
+int prologue_groups(const PrologueParams& pp) {
+    const int64_t heads = (int64_t)pp.B * pp.Hkv;
+    return (int)std::max<int64_t>(1, std::min<int64_t>((pp.wq + 63) / 64, 2 * device_cu_count() / heads));
 }
 
 // ---------------------------------------------------------------------------
@@ -3029,7 +3055,11 @@ int latent_decode_run(const slimkv_latent_decode_args* a, const PagedRows* pg, v
         else if (nct == 2) hipLaunchKernelGGL(prologue_mfma_kernel<2>, dim3(B * Hkv), dim3(64), 0, st, pp);
         else hipLaunchKernelGGL(prologue_mfma_kernel<3>, dim3(B * Hkv), dim3(64), 0, st, pp);
     } else if (has_lat && g * Lq <= 16 && ptr_aligned16(a->q) && ptr_aligned16(a->up_k) && (!pp.shift || ptr_aligned16(a->up_k_bias))) {
-        hipLaunchKernelGGL(prologue_wide_kernel, dim3(B * Hkv * ((pp.wq + 63) / 64)), dim3(256), 0, st, pp);
+        const int groups = prologue_groups(pp);
+        if (groups == (pp.wq + 63) / 64)
+            hipLaunchKernelGGL(prologue_wide_kernel<false>, dim3(B * Hkv * groups), dim3(256), 0, st, pp, groups);
+        else
+            hipLaunchKernelGGL(prologue_wide_kernel<true>, dim3(B * Hkv * groups), dim3(256), 0, st, pp, groups);
     } else {
         hipLaunchKernelGGL(prologue_kernel, dim3(B * Hkv), dim3(256), 0, st, pp);
     }

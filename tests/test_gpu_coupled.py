@@ -112,6 +112,11 @@ SIZES = [(1, 32, 8, 1, 5, 256, 256, 1, False), (2, 32, 8, 63, 133, 128, 64, 1, T
          (2, 96, 8, 333, 17, 384, 384, 1, False), (1, 64, 8, 129, 33, 64, 120, 2, False)]
 
 
+# several blocks of 64 columns to a workgroup of the query absorption: two or
+# three of five, all of three, with a last block of 8 and of 64 columns
+SIZES += [(22, 32, 8, 40, 5, 320, 200, 1, True), (70, 8, 8, 30, 5, 136, 72, 2, True)]
+
+
 @pytest.mark.parametrize('B,Hq,Hkv,n,raw,rk,rv,queries,bias', SIZES)
 def test_sizes(device, B, Hq, Hkv, n, raw, rk, rv, queries, bias):
     check(layer(device, B, Hq, Hkv, n, raw, rk, rv, queries, bias), f'{n} beacons')

@@ -2094,13 +2094,13 @@ struct PrologueParams {
     int blockdiag; int wq;                 // q_lat width (own block or Rk)
     uint16_t* q_lat;                       // [B][Lq][Hq][wq]
     float* shift;                          // [B][Hq*Lq] or null
-    int B, Lq, Hq, Hkv, D, Rk, parts;      // parts: power of two <= 16 dividing D
+    int bias16;                            // up_k_bias on a 16-byte boundary
+    int B, Lq, Hq, Hkv, D, Rk;
     float scale;
     const uint16_t* ut;                    // [Hkv][wq][D] per-head U_K^T (MFMA prologue) or null
 };
 
 constexpr int kMaxRows = 16;
-constexpr int kMaxD = 256;
 
 // RoPE table row of query (b, l): its position, or -- without positions --
 // row b * Lq + l of tables already taken at the query positions (one gather
@@ -2110,118 +2110,39 @@ __device__ __forceinline__ int64_t query_rope_row(const PrologueParams& pp, int 
     return clamp_i64(pp.pos[(int64_t)b * pp.pos_sb + l], 0, pp.rope_rows - 1);
 }
 
-// One workgroup per (b, KV head).  Rows r = jj*Lq + l of the head's query group
-// are rotated into LDS; thread (k8, part) then forms 8 consecutive q_lat
-// columns over a D/parts slice with 16-byte weight loads, and the parts are
-// reduced with lane shuffles (they are adjacent lanes).
+// Calls without beacon rows: the query rows of a (b, KV head) rotated into the
+// workspace, 8 elements a thread.
 __global__ void __launch_bounds__(256)
 prologue_kernel(PrologueParams pp) {
-    __shared__ float qs[kMaxRows * kMaxD];
+    constexpr int D = 128, HALF = D / 2, PIECES = D / 8;
     const int h = blockIdx.x % pp.Hkv;
     const int b = blockIdx.x / pp.Hkv;
     const int g = pp.Hq / pp.Hkv;
-    const int rows = g * pp.Lq;
-    const int D = pp.D;
-    const int pieces = D / 8;
-    for (int e = threadIdx.x; e < rows * pieces; e += blockDim.x) {
-        const int r = e / pieces, dd = (e % pieces) * 8;
-        const int jj = r / pp.Lq, l = r % pp.Lq;
-        const int jh = h * g + jj;
-        const uint16_t* qrow = pp.q + (int64_t)b * pp.q_sb + (int64_t)l * pp.q_sl + (int64_t)jh * pp.q_sh;
-        const u32x4 xv = *reinterpret_cast<const u32x4*>(qrow + dd);
-        uint32_t xs[4] = {xv.x, xv.y, xv.z, xv.w};
-        float x[8];
+    const int e = threadIdx.x;              // at most kMaxRows * PIECES = 256 of them
+    if (e >= g * pp.Lq * PIECES) return;
+    const int r = e / PIECES, dd = e % PIECES * 8;
+    const int j = h * g + r / pp.Lq, l = r % pp.Lq;
+    const uint16_t* qrow = pp.q + (int64_t)b * pp.q_sb + (int64_t)l * pp.q_sl + (int64_t)j * pp.q_sh;
+    u32x4 x = *reinterpret_cast<const u32x4*>(qrow + dd);
+    if (pp.cos) {
+        const u32x4 y = *reinterpret_cast<const u32x4*>(qrow + (dd < HALF ? dd + HALF : dd - HALF));
+        const int64_t pos = query_rope_row(pp, b, l);
+        const float4* c4 = reinterpret_cast<const float4*>(pp.cos + pos * D + dd);
+        const float4* s4 = reinterpret_cast<const float4*>(pp.sin + pos * D + dd);
+        const float4 ca = c4[0], cb = c4[1], sa = s4[0], sb = s4[1];
+        const float cs[8] = {ca.x, ca.y, ca.z, ca.w, cb.x, cb.y, cb.z, cb.w};
+        const float ss[8] = {sa.x, sa.y, sa.z, sa.w, sb.x, sb.y, sb.z, sb.w};
+        const float sign = dd < HALF ? -1.f : 1.f;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            x[2 * i] = bf16_to_f32(xs[i] & 0xffffu);
-            x[2 * i + 1] = bf16_to_f32(xs[i] >> 16);
+            const float o0 = round_bf16_hw(lo_bf16(x[i]) * round_bf16_hw(cs[2 * i])) +
+                             round_bf16_hw(sign * lo_bf16(y[i]) * round_bf16_hw(ss[2 * i]));
+            const float o1 = round_bf16_hw(hi_bf16(x[i]) * round_bf16_hw(cs[2 * i + 1])) +
+                             round_bf16_hw(sign * hi_bf16(y[i]) * round_bf16_hw(ss[2 * i + 1]));
+            x[i] = pack_bf16(o0, o1);
         }
-        if (pp.cos) {
-            const int half = D / 2;
-            const int pd = dd < half ? dd + half : dd - half;
-            const u32x4 pv = *reinterpret_cast<const u32x4*>(qrow + pd);
-            const uint32_t ps[4] = {pv.x, pv.y, pv.z, pv.w};
-            const int64_t pos = query_rope_row(pp, b, l);
-            const float4* c4 = reinterpret_cast<const float4*>(pp.cos + pos * D + dd);
-            const float4* s4 = reinterpret_cast<const float4*>(pp.sin + pos * D + dd);
-            const float4 ca = c4[0], cb = c4[1], sa = s4[0], sb = s4[1];
-            const float cs[8] = {ca.x, ca.y, ca.z, ca.w, cb.x, cb.y, cb.z, cb.w};
-            const float ss[8] = {sa.x, sa.y, sa.z, sa.w, sb.x, sb.y, sb.z, sb.w};
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                float pt = bf16_to_f32(i & 1 ? (ps[i / 2] >> 16) : (ps[i / 2] & 0xffffu));
-                if (dd < half) pt = -pt;
-                x[i] = round_bf16_hw(round_bf16_hw(x[i] * round_bf16_hw(cs[i])) +
-                                     round_bf16_hw(pt * round_bf16_hw(ss[i])));
-            }
-#pragma unroll
-            for (int i = 0; i < 4; ++i) xs[i] = pack_bf16(x[2 * i], x[2 * i + 1]);
-        }
-#pragma unroll
-        for (int i = 0; i < 8; ++i) qs[r * D + dd + i] = x[i];
-        *reinterpret_cast<u32x4*>(pp.q_rot + (((int64_t)b * pp.Lq + l) * pp.Hq + jh) * D + dd) =
-            u32x4{xs[0], xs[1], xs[2], xs[3]};
     }
-    __syncthreads();
-    if (pp.shift && threadIdx.x < rows) {
-        const int r = threadIdx.x;
-        const int jj = r / pp.Lq, l = r % pp.Lq;
-        float sum = 0.f;
-        for (int dd = 0; dd < D; ++dd)
-            sum += qs[r * D + dd] * bf16_to_f32(pp.up_k_bias[(int64_t)h * D + dd]);
-        pp.shift[(int64_t)b * pp.Hq * pp.Lq + (h * g + jj) * pp.Lq + l] = sum * pp.scale;
-    }
-    if (pp.wq == 0) return;
-    // Absorption: thread (row r, 8-column group k8, part) sums D/parts terms for
-    // 8 consecutive q_lat columns; partial sums meet in LDS.
-    __shared__ float red[256 * 8];
-    const int parts = pp.parts;
-    const int per = D / parts;
-    const int k8n = pp.wq / 8;
-    for (int base = 0; base < rows * k8n * parts; base += 256) {
-        const int task = base + threadIdx.x;
-        const bool active = task < rows * k8n * parts;
-        const int part = task % parts;
-        const int rk = task / parts;            // r * k8n + k8
-        const int r = rk / k8n, k8 = rk % k8n;
-        float acc8[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-        if (active) {
-            const int kg = (pp.blockdiag ? h * pp.wq : 0) + 8 * k8;
-            const uint16_t* wbase = pp.up_k + ((int64_t)h * D + part * per) * pp.Rk + kg;
-            const float* qr = qs + r * D + part * per;
-            for (int d0 = 0; d0 < per; d0 += 8) {
-                u32x4 wv[8];
-#pragma unroll
-                for (int i = 0; i < 8; ++i) wv[i] = *reinterpret_cast<const u32x4*>(wbase + (int64_t)(d0 + i) * pp.Rk);
-#pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    const float qv = qr[d0 + i];
-                    const uint32_t w4[4] = {wv[i].x, wv[i].y, wv[i].z, wv[i].w};
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        acc8[2 * e] += qv * bf16_to_f32(w4[e] & 0xffffu);
-                        acc8[2 * e + 1] += qv * bf16_to_f32(w4[e] >> 16);
-                    }
-                }
-            }
-        }
-#pragma unroll
-        for (int e = 0; e < 8; ++e) red[threadIdx.x * 8 + e] = acc8[e];
-        __syncthreads();
-        if (active && part == 0) {
-            float sum[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-            for (int q = 0; q < parts; ++q)
-#pragma unroll
-                for (int e = 0; e < 8; ++e) sum[e] += red[(threadIdx.x + q) * 8 + e];
-            const int jj = r / pp.Lq, l = r % pp.Lq;
-            uint32_t o4[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) o4[e] = pack_bf16(sum[2 * e], sum[2 * e + 1]);
-            *reinterpret_cast<u32x4*>(pp.q_lat + (((int64_t)b * pp.Lq + l) * pp.Hq + h * g + jj) * pp.wq + 8 * k8) =
-                u32x4{o4[0], o4[1], o4[2], o4[3]};
-        }
-        __syncthreads();
-    }
+    *reinterpret_cast<u32x4*>(pp.q_rot + (((int64_t)b * pp.Lq + l) * pp.Hq + j) * D + dd) = x;
 }
 
 // MFMA prologue for block-diagonal bases, one wavefront per (b, KV head): the
@@ -2343,7 +2264,14 @@ prologue_wide_kernel(PrologueParams pp, int groups) {
         if (pp.shift && first) {
             const uint16_t* bk = pp.up_k_bias + (int64_t)h * D + 8 * grp;
 #pragma unroll
-            for (int c = 0; c < 4; ++c) kb[c] = *reinterpret_cast<const u32x4*>(bk + 32 * c);
+            for (int c = 0; c < 4; ++c) {
+                if (pp.bias16) {
+                    kb[c] = *reinterpret_cast<const u32x4*>(bk + 32 * c);
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) kb[c][e] = bk[32 * c + 2 * e] | (uint32_t)bk[32 * c + 2 * e + 1] << 16;
+                }
+            }
         }
         stage();
 #pragma unroll
@@ -2706,10 +2634,9 @@ struct LatentPlan {
     int coupled;          // latent rows by the coupled kernel: groups of 16 query rows a workgroup, 0 = split kernel
     int groups;           // workgroups that share a sequence's query rows there
     int wq;               // q_lat width per head
-    int parts;
+    bool bases;           // the absorption reads the prepared transposed bases (up_k_t), else up_k
     size_t qrot_off, qlat_off, shift_off, rml_off, racc_off, lml_off, lacc_off, total;
     size_t bound;         // workspace asked for: total, or more where the header promises it for other sizes
-    size_t prologue_lds;
 };
 
 // Beacon rows read straight out of pages (slimkv_paged_latent_decode).
@@ -2791,7 +2718,7 @@ int plan_latent(const slimkv_latent_decode_args* a, LatentPlan* p, const PagedRo
                                a->rv_sh, a->lk_sb, a->lk_sn, a->lv_sb, a->lv_sn};
     for (int64_t st : strides)
         if (!aligned8(st)) return fail(SLIMKV_EINVAL, "strides must be multiples of 8 elements");
-    if (!ptr_aligned16(a->raw_k) || !ptr_aligned16(a->raw_v) || !ptr_aligned16(a->lat_k) ||
+    if (!ptr_aligned16(a->q) || !ptr_aligned16(a->raw_k) || !ptr_aligned16(a->raw_v) || !ptr_aligned16(a->lat_k) ||
         !ptr_aligned16(a->lat_v) || !ptr_aligned16(a->up_v))
         return fail(SLIMKV_EINVAL, "tensors must be 16-byte aligned");
     const bool bd = a->block_diagonal != 0;
@@ -2799,6 +2726,9 @@ int plan_latent(const slimkv_latent_decode_args* a, LatentPlan* p, const PagedRo
         return fail(SLIMKV_EINVAL, "block-diagonal ranks must split into per-head multiples of 8");
     const int rk = (int)(bd ? Rk / Hkv : Rk);
     const int rv = (int)(bd ? Rv / Hkv : Rv);
+    p->bases = a->lat_keys > 0 && bd && a->up_k_t && rk % 16 == 0 && rk <= 48 && ptr_aligned16(a->up_k_t) &&
+               ptr_aligned16(a->up_k_bias);
+    if (a->lat_keys > 0 && !p->bases && !ptr_aligned16(a->up_k)) return fail(SLIMKV_EINVAL, "tensors must be 16-byte aligned");
     const int cu = device_cu_count();
     // Latent: every query head against shared rows.  With block-diagonal bases a
     // tile spans only its own heads' latent slices; narrow tiles (8 packed rows)
@@ -2965,10 +2895,6 @@ int plan_latent(const slimkv_latent_decode_args* a, LatentPlan* p, const PagedRo
         p->lat.nwg = wave_item_groups((int)B, p->lat.splits, p->lat.tiles);
     }
     p->wq = rk;
-    int parts = 1;
-    while (parts < 16 && g * (int)Lq * (p->wq / 8) * parts * 2 <= 256) parts *= 2;
-    p->parts = parts;
-    p->prologue_lds = 0;
     size_t off = 0;
     p->qrot_off = off; off = align256(off + (size_t)B * Lq * Hq * D * 2);
     p->qlat_off = off; off = align256(off + (size_t)B * Lq * Hq * p->wq * 2);
@@ -3034,27 +2960,25 @@ int latent_decode_run(const slimkv_latent_decode_args* a, const PagedRows* pg, v
     pp.wq = has_lat ? p.wq : 0;
     pp.q_lat = q_lat;
     pp.shift = (has_lat && a->up_k_bias) ? shift : nullptr;
-    pp.B = B; pp.Lq = Lq; pp.Hq = Hq; pp.Hkv = Hkv; pp.D = D; pp.Rk = Rk; pp.parts = p.parts;
+    pp.bias16 = ptr_aligned16(a->up_k_bias);
+    pp.B = B; pp.Lq = Lq; pp.Hq = Hq; pp.Hkv = Hkv; pp.D = D; pp.Rk = Rk;
     pp.scale = (float)a->scale;
     pp.ut = static_cast<const uint16_t*>(a->up_k_t);
     const int nct = pp.wq / 16;
-    const bool mfma_prologue = has_lat && bd && pp.ut && pp.wq % 16 == 0 && nct >= 1 && nct <= 3 &&
-                               g * Lq <= 16 && ptr_aligned16(pp.ut) && ptr_aligned16(a->q) &&
-                               (!a->up_k_bias || ptr_aligned16(a->up_k_bias));
     // With per-head bases, a call that runs the prologue and the attend stage
     // together makes the query operands inside the split kernel (its raw waves
     // rotate their rows and, with a K bias, write the rows' LSE shifts; its
     // latent waves rotate and absorb theirs): two launches a layer instead of
     // three, the same bits.
-    const bool fused = mfma_prologue && (stages & SLIMKV_STAGE_PROLOGUE) && (stages & SLIMKV_STAGE_ATTEND) &&
+    const bool fused = p.bases && (stages & SLIMKV_STAGE_PROLOGUE) && (stages & SLIMKV_STAGE_ATTEND) &&
                        split_fq_ok(p.lat.ks, pg != nullptr, pg ? (int)pg->slots : 0);
     if (fused || !(stages & SLIMKV_STAGE_PROLOGUE)) {
         // the query operands of an earlier prologue stage are in the workspace
-    } else if (mfma_prologue) {
+    } else if (p.bases) {
         if (nct == 1) hipLaunchKernelGGL(prologue_mfma_kernel<1>, dim3(B * Hkv), dim3(64), 0, st, pp);
         else if (nct == 2) hipLaunchKernelGGL(prologue_mfma_kernel<2>, dim3(B * Hkv), dim3(64), 0, st, pp);
         else hipLaunchKernelGGL(prologue_mfma_kernel<3>, dim3(B * Hkv), dim3(64), 0, st, pp);
-    } else if (has_lat && g * Lq <= 16 && ptr_aligned16(a->q) && ptr_aligned16(a->up_k) && (!pp.shift || ptr_aligned16(a->up_k_bias))) {
+    } else if (has_lat) {
         const int groups = prologue_groups(pp);
         if (groups == (pp.wq + 63) / 64)
             hipLaunchKernelGGL(prologue_wide_kernel<false>, dim3(B * Hkv * groups), dim3(256), 0, st, pp, groups);
@@ -3333,6 +3257,8 @@ int plan_recon(const slimkv_recon_decode_args* r, ReconPlan* p) {
     if (B <= 0 || Lq <= 0 || Lq > 2 || Hq <= 0 || Hkv <= 0 || Hq % Hkv) return fail(SLIMKV_EINVAL, "invalid sizes");
     if (D != 128) return fail(SLIMKV_EUNSUP, "reconstruction decode is built for head_dim 128");
     if (a->raw_keys <= 0 || a->lat_keys < 0) return fail(SLIMKV_EINVAL, "invalid key counts");
+    if (!ptr_aligned16(a->q) || !aligned8(a->q_sb) || !aligned8(a->q_sl) || !aligned8(a->q_sh))
+        return fail(SLIMKV_EINVAL, "query rows must be 16-byte aligned");
     if (a->lat_keys > 0 && (!a->lat_k || !a->lat_v)) return fail(SLIMKV_EINVAL, "null latent pointer");
     if (r->beacon_positions && B > 1 && r->bpos_sb < a->lat_keys)
         return fail(SLIMKV_EINVAL, "beacon position rows are shorter than the beacon count");

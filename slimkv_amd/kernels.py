@@ -37,6 +37,11 @@ def _last_contiguous(t):
     return t if t.stride(-1) == 1 else t.contiguous()
 
 
+def _aligned(t):
+    """t, or a copy of it where its rows start off a 16-byte boundary."""
+    return t if t.data_ptr() % 16 == 0 else t.clone(memory_format=torch.contiguous_format)
+
+
 def _int64(t):
     return t if t.dtype is torch.int64 else t.to(torch.int64)
 
@@ -273,9 +278,9 @@ def _latent_rows(lat_k, lat_v, Rk, Rv):
 
 def _latent_args(q, raw_k, raw_v, lat_k, lat_v, up_k, up_v, scale, up_k_bias, up_v_bias, block_diagonal,
                  lat_causal, q_positions, cos, sin, raw_lengths, lat_lengths, raw_splits, lat_splits, out, lse,
-                 prepared_bases=True, lat_rows=None, lat_k2=None, lat_v2=None, raw_shape=None):
+                 prepared_bases=True, lat_rows=None, lat_k2=None, lat_v2=None, raw_shape=None, absorb=True):
     """raw_shape = (raw rows, KV heads) when the raw rows are read through raw
-    pages (raw_k / raw_v None)."""
+    pages (raw_k / raw_v None).  absorb: the queries are absorbed into up_k."""
     _need_device(q, raw_k, raw_v, lat_k, lat_v, lat_k2, lat_v2, up_k, up_v)
     _need_bf16(q, raw_k, raw_v, lat_k, lat_v, lat_k2, lat_v2, up_k, up_v, up_k_bias, up_v_bias)
     B, Lq, Hq, D = q.shape
@@ -288,7 +293,7 @@ def _latent_args(q, raw_k, raw_v, lat_k, lat_v, up_k, up_v, scale, up_k_bias, up
         lat_k, lat_v, lat_k2, lat_v2 = lat_k2, lat_v2, None, None
     Nl = (0 if lat_rows is None else int(lat_rows)) if lat_k is None else lat_k.shape[1]
     split = 0
-    q = _last_contiguous(q)
+    q = _aligned(_last_contiguous(q))
     if raw_k is not None:
         raw_k, raw_v = _last_contiguous(raw_k), _last_contiguous(raw_v)
     if lat_k is not None:
@@ -320,6 +325,9 @@ def _latent_args(q, raw_k, raw_v, lat_k, lat_v, up_k, up_v, scale, up_k_bias, up
     if prepared_bases and block_diagonal and Nl > 0 and Rk % Hkv == 0 \
             and (Rk // Hkv) % 16 == 0 and D == 128:
         bases = prepare_latent_bases(up_k, Hkv)
+    if absorb and up_k.data_ptr() % 16 and (bases is None or Rk // Hkv > 48 or
+                                            (up_k_bias is not None and up_k_bias.data_ptr() % 16)):
+        up_k = _aligned(up_k)            # the absorption then reads up_k itself
     a = _lib.LatentDecodeArgs(
         _ptr(q), *q.stride()[:3],
         _ptr(q_positions), 0 if q_positions is None else q_positions.stride(0),
@@ -580,9 +588,12 @@ def recon_decode(q, raw_k, raw_v, lat_k, lat_v, up_k, up_v, scale, *, beacon_pos
     rotated beacon keys are rebuilt in fp32 and rounded once, unless
     reference_rounding asks for the reference's bf16 steps (the bits
     ReconstructionCache.materialize writes, modeling_llama.py:1405-1483)."""
+    if any(s % 8 for s in q.stride()[:3]):
+        q = q.contiguous()
     base, out, lse, keep = _latent_args(q, raw_k, raw_v, lat_k, lat_v, up_k, up_v, scale, up_k_bias, up_v_bias,
                                         block_diagonal, lat_causal, q_positions, cos, sin, raw_lengths,
-                                        lat_lengths, raw_splits, lat_splits, out, lse, prepared_bases=False)
+                                        lat_lengths, raw_splits, lat_splits, out, lse, prepared_bases=False,
+                                        absorb=False)
     pairs = None
     if beacon_positions is not None:
         beacon_positions = _int64(beacon_positions)

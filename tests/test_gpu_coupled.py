@@ -250,3 +250,61 @@ def test_device_scratch_gives_the_bits_of_a_workspace(device, B, n, raw, lat_spl
     _lib.check(_lib.lib().slimkv_latent_decode_noalloc(ctypes.byref(a), _lib.stream_handle(device)))
     torch.cuda.synchronize()
     assert torch.equal(got, want) and torch.equal(got_lse, want_lse)
+
+
+def _shifted(t, by):
+    """The values of t, starting `by` elements past a 16-byte boundary."""
+    flat = torch.empty(t.numel() + by, dtype=t.dtype, device=t.device)[by:].view(t.shape)
+    return flat.copy_(t)
+
+
+@pytest.mark.parametrize('rank', [64, 128, 256])
+@pytest.mark.parametrize('per_head', [False, True])
+def test_operands_off_a_16_byte_boundary_give_the_same_bits(device, per_head, rank):
+    """Queries, U_K and the K bias may start anywhere: copied, or read
+    narrowly."""
+    from slimkv_amd import kernels
+    from slimkv_amd.workloads import block_diagonal
+    args, kw, *_ = layer(device, 2, 32, 8, 300, 21, rank, rank, bias=True)
+    q, rk, rv, lk, lv, uk, uv, scale = args
+    if per_head:
+        r = rank // 8
+        uk, uv = (block_diagonal([t[128 * h:128 * h + 128, :r] for h in range(8)]) for t in (uk, uv))
+    kw['block_diagonal'] = per_head
+    want = kernels.latent_decode(q, rk, rv, lk, lv, uk, uv, scale, prepared_bases=False, **kw)
+    for moved in ('q', 'up_k', 'bias'):
+        got = kernels.latent_decode(_shifted(q, 4) if moved == 'q' else q, rk, rv, lk, lv,
+                                    _shifted(uk, 1) if moved == 'up_k' else uk, uv, scale, prepared_bases=False,
+                                    **dict(kw, up_k_bias=_shifted(kw['up_k_bias'], 3) if moved == 'bias' else kw['up_k_bias']))
+        assert all(torch.equal(x, y) for x, y in zip(got, want)), moved
+    if per_head:
+        want = kernels.latent_decode(q, rk, rv, lk, lv, uk, uv, scale, **kw)
+        got = kernels.latent_decode(_shifted(q, 4), rk, rv, lk, lv, _shifted(uk, 1), uv, scale, **kw)
+        assert all(torch.equal(x, y) for x, y in zip(got, want))
+    if per_head and rank == 64:
+        return                              # the rebuild takes multiples of 16
+    odd = torch.empty(2, 1, 32, 132, dtype=q.dtype, device=device)[..., 4:].copy_(q)
+    recon = [kernels.recon_decode(x, rk, rv, lk, lv, uk, uv, scale, **kw) for x in (q, _shifted(q, 1), odd)]
+    assert all(torch.equal(x, y) for other in recon[1:] for x, y in zip(other, recon[0]))
+
+
+@pytest.mark.parametrize('queries,positions', [(1, True), (2, True), (2, False)])
+def test_raw_rows_alone(device, queries, positions):
+    """No beacons: the queries are rotated for the raw rows only."""
+    from slimkv_amd import kernels
+    args, kw, *_ = layer(device, 3, 40, 8, 8, 77, 64, 64, queries)
+    q, rk, rv, _, _, uk, uv, scale = args
+    cos, sin, pos = kw['cos'], kw['sin'], kw['q_positions']
+    rope = dict(cos=cos, sin=sin, q_positions=pos)
+    if not positions:
+        rows = kernels.query_rope_rows(cos, sin, pos)
+        rope = dict(cos=rows[0], sin=rows[1])
+    empty = torch.empty(3, 0, 64, dtype=q.dtype, device=device)
+    got, lse = kernels.latent_decode(q, rk, rv, empty, empty, uk, uv, scale, **rope)
+    c, s = (t.to(torch.bfloat16).double()[pos][:, :, None] for t in (cos, sin))
+    x = q.double()
+    x = (x * c + torch.cat([-x[..., 64:], x[..., :64]], -1) * s).view(3, queries, 8, 5, D).permute(0, 2, 3, 1, 4)
+    k, v = (t.double().permute(0, 2, 1, 3)[:, :, None] for t in (rk, rv))
+    sc = torch.matmul(x, k.transpose(-1, -2).contiguous()) * scale
+    want = torch.matmul(torch.softmax(sc, -1), v).permute(0, 3, 1, 2, 4).reshape(3, queries, 40, D)
+    assert_close(to_np(got), want.cpu().numpy(), max_abs=max(MAX_ABS, 2.0 ** -7 * float(want.abs().max())), what='raw rows')

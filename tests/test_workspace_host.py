@@ -73,3 +73,29 @@ def test_the_device_scratch_holds_coupled_partials(batch, heads, queries, rank_v
         rows = batch * heads * queries
         for n, size in enumerate(given, 1):
             assert size <= given[0] + (n - 1) * rows * (4 * rank_v + 8) + 512
+
+
+def test_rows_off_a_16_byte_boundary_are_refused():
+    """Operands that the kernels read 16 bytes at a time; U_K only where the
+    absorption reads it (not the prepared bases of per-head ones)."""
+    from slimkv_amd import _lib
+    lib = _lib.lib()
+    for name in ('q', 'raw_k', 'lat_v', 'up_k', 'up_v'):
+        a = latent_args(1, 32, 700, 256, 256)
+        setattr(a, name, (1 << 20) + 8)
+        assert lib.slimkv_latent_decode_workspace(ctypes.byref(a)) == 0, name
+        assert b'16-byte' in lib.slimkv_last_error()
+    a = latent_args(1, 32, 700, 256, 256, per_head=True)
+    a.up_k = (1 << 20) + 8
+    assert lib.slimkv_latent_decode_workspace(ctypes.byref(a)) == 0
+    a.up_k_t = 1 << 20
+    assert lib.slimkv_latent_decode_workspace(ctypes.byref(a)) > 0
+    a.up_k_bias = (1 << 20) + 2
+    assert lib.slimkv_latent_decode_workspace(ctypes.byref(a)) == 0
+    for change in ({'q': (1 << 20) + 8}, {'q_sh': 132}):
+        r = _lib.ReconDecodeArgs()
+        r.base = latent_args(1, 32, 700, 256, 256)
+        assert lib.slimkv_recon_decode_workspace(ctypes.byref(r)) > 0
+        for name, value in change.items():
+            setattr(r.base, name, value)
+        assert lib.slimkv_recon_decode_workspace(ctypes.byref(r)) == 0

@@ -43,7 +43,7 @@ extern "C" {
 /* Message describing the last failure on the calling thread ("" if none). */
 const char* slimkv_last_error(void);
 
-/* ABI version of this header (bumped on any struct change). */
+/* ABI version of this header: raised with any struct, constant or entry point. */
 int slimkv_abi_version(void);
 
 /* Stages of a decode call, for the *_stages entry points (bit mask).  A

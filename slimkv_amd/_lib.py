@@ -279,7 +279,7 @@ SIGNATURES = {
     'slimkv_paged_step_rows': (ctypes.c_int, [ctypes.POINTER(PagedStepRowsArgs), c_ptr]),
 }
 
-ABI_VERSION = 15
+ABI_VERSION = 16
 
 STAGE_PROLOGUE, STAGE_ATTEND, STAGE_COMBINE, STAGE_ALL = 1, 2, 4, 7
 NOALLOC_SCRATCH_BYTES = 64 << 20

@@ -87,6 +87,17 @@ def test_struct_offsets_match_the_c_compiler(tmp_path):
     assert got[:-1] == want
 
 
+def test_the_abi_number_moves_with_the_declared_interface():
+    """The number that the binding asks for and the interface it stands for: a
+    change of either without the other fails here."""
+    import hashlib
+    from slimkv_amd import _lib
+    text = re.sub(r'/\*.*?\*/', '', (ROOT / 'include' / 'slimkv_hip.h').read_text(), flags=re.S)
+    digest = hashlib.sha256(' '.join(text.split()).encode()).hexdigest()[:12]
+    assert (_lib.ABI_VERSION, digest) == (16, 'd73c845410f8')
+    assert _lib.lib().slimkv_abi_version() == _lib.ABI_VERSION
+
+
 def test_errors_are_reported_without_a_gpu():
     from slimkv_amd import _lib
     a = _lib.AttentionArgs()

@@ -510,8 +510,10 @@ template <int KS, int RT>
 hipError_t launch_wide_rt(const ReconParams& p, int segs, hipStream_t st) {
     const dim3 grid(p.B * p.Hkv * segs), block(kReconWaves * 64);
     if (p.positions) {
-        if (p.in16) hipLaunchKernelGGL((recon_wide_kernel<KS, RT, true, true>), grid, block, 0, st, p, segs);
-        else hipLaunchKernelGGL((recon_wide_kernel<KS, RT, true, false>), grid, block, 0, st, p, segs);
+        if constexpr (KS < 16 || RT == 1) {                // width 512 with RoPE has one row group (prepare_recon)
+            if (p.in16) hipLaunchKernelGGL((recon_wide_kernel<KS, RT, true, true>), grid, block, 0, st, p, segs);
+            else hipLaunchKernelGGL((recon_wide_kernel<KS, RT, true, false>), grid, block, 0, st, p, segs);
+        }
     } else {
         if (p.in16) hipLaunchKernelGGL((recon_wide_kernel<KS, RT, false, true>), grid, block, 0, st, p, segs);
         else hipLaunchKernelGGL((recon_wide_kernel<KS, RT, false, false>), grid, block, 0, st, p, segs);
@@ -647,12 +649,13 @@ hipError_t launch_wide_pair(const ReconParams& p0, int segs0, const ReconParams&
     const dim3 grid(blocks0 + blocks1), block(kReconWaves * 64);
 #define SLIMKV_PAIR(RT, ROPE) \
     hipLaunchKernelGGL((recon_wide_pair_kernel<KS, RT, ROPE>), grid, block, 0, st, p0, p1, segs0, segs1, blocks0)
-    if (p0.positions) {
-        if (p0.row_frags == 1) SLIMKV_PAIR(1, true);
-        else SLIMKV_PAIR(2, true);
+    if (p0.row_frags == 1) {
+        if (p0.positions) SLIMKV_PAIR(1, true);
+        else SLIMKV_PAIR(1, false);
+    } else if (!p0.positions) {
+        SLIMKV_PAIR(2, false);
     } else {
-        if (p0.row_frags == 1) SLIMKV_PAIR(1, false);
-        else SLIMKV_PAIR(2, false);
+        if constexpr (KS < 16) SLIMKV_PAIR(2, true);       // width 512 with RoPE has one row group (prepare_recon)
     }
 #undef SLIMKV_PAIR
     return hipGetLastError();
@@ -660,7 +663,7 @@ hipError_t launch_wide_pair(const ReconParams& p0, int segs0, const ReconParams&
 
 int reconstruct_pair(const slimkv_reconstruct_args* a, const slimkv_reconstruct_args* b, hipStream_t st,
                      const uint32_t* pairs, int repeats) {
-    ReconParams pa, pb;
+    ReconParams pa{}, pb{};
     int sa = 0, sb = 0, ka = 0, kb = 0;
     int rc = prepare_recon(a, &pa, &sa, &ka);
     if (rc != SLIMKV_OK) return rc;

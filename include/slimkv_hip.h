@@ -542,7 +542,9 @@ int slimkv_prefill_attention(const slimkv_prefill_attention_args* a, void* strea
 /* The same call with a workspace of slimkv_prefill_attention_workspace(a)
  * bytes (16-byte aligned; 0: none is used): few long query blocks are then
  * split over their keys so that every CU ends at the same time, and merged in
- * fp32.  With a smaller workspace the call runs unsplit. */
+ * fp32.  The size is two entries of 66,560 bytes for each of two workgroups a
+ * CU (65 MiB on 256 CUs), whatever the call.  With a smaller workspace the call
+ * runs unsplit. */
 size_t slimkv_prefill_attention_workspace(const slimkv_prefill_attention_args* a);
 int slimkv_prefill_attention_split(const slimkv_prefill_attention_args* a, void* workspace, size_t workspace_bytes,
                                    void* stream);

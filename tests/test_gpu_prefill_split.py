@@ -46,6 +46,51 @@ def test_split_schedule(device, B, Hq, Hkv, L, N, causal):
         assert_close(to_np(out[b, rows, h]), (torch.softmax(sc, -1) @ vv).cpu().numpy(), what=f'head {h}')
 
 
+@pytest.mark.parametrize('repeats', [True, False])
+@pytest.mark.parametrize('B,Hq,Hkv,L,N', [(1, 32, 8, 1280, 9220), (3, 20, 4, 300, 18000)])
+def test_split_over_the_kept_set_with_query_rope(device, B, Hq, Hkv, L, N, repeats):
+    """The window attention as the package calls it: K and V views of a kept
+    [B, Hkv, capacity, D] set, queries of a [B, Hq, L, D] projection rotated at
+    their positions from prepared pairs, rows that repeat their first half and
+    rows that do not."""
+    from slimkv_amd import _lib, kernels
+    from slimkv_amd.workloads import rope_tables
+    gen = torch.Generator(device=device).manual_seed(L + N)
+
+    def rnd(*shape):
+        return torch.randn(*shape, generator=gen, device=device).to(torch.bfloat16)
+    q = rnd(B, Hq, L, D).transpose(1, 2)
+    k, v = (rnd(B, Hkv, N + 700, D)[:, :, :N].transpose(1, 2) for _ in range(2))
+    cos, sin = rope_tables(N + 50, D, 500000.0, device)
+    if not repeats:
+        cos, sin = (torch.cat([t[:, :64], t[:, 64:].roll(7, 0)], 1).contiguous() for t in (cos, sin))
+    pos = (torch.arange(L, device=device) + N - L + 37)[None].expand(B, -1)
+    out, lse = kernels.prefill_attention(q, k, v, D ** -0.5, q_positions=pos, cos=cos, sin=sin)
+    pairs, same = kernels.prepare_rope_pairs(cos, sin)
+    assert bool(same) == repeats
+    plain, plain_lse = torch.empty_like(out), torch.empty_like(lse)
+    a = _lib.PrefillAttentionArgs(q.data_ptr(), *q.stride()[:3], k.data_ptr(), *k.stride()[:3], v.data_ptr(),
+                                  *v.stride()[:3], plain.data_ptr(), *plain.stride()[:3], plain_lse.data_ptr(), None,
+                                  B, L, Hq, Hkv, N, D, D ** -0.5, 1, pairs.data_ptr(), pairs.shape[0], int(same),
+                                  pos.data_ptr(), pos.stride(0))
+    assert _lib.lib().slimkv_prefill_attention_workspace(ctypes.byref(a)) > 0
+    _lib.check(_lib.lib().slimkv_prefill_attention(ctypes.byref(a), _lib.stream_handle(device)))
+    # as above: both results round their probabilities against other maxima
+    weight = kernels.prefill_attention(q, k, v.abs(), D ** -0.5, q_positions=pos, cos=cos, sin=sin)[0].float()
+    diff = (out.float() - plain.float()).abs()
+    assert bool((diff <= 2.0 ** -7 * weight + 2.0 ** -8 * plain.float().abs()).all())
+    assert_lse_close(to_np(lse), to_np(plain_lse), atol=2.0 ** -8)
+    c, s = (t.to(torch.bfloat16).double()[pos[0]] for t in (cos, sin))
+    for b, h in ((0, 0), (B - 1, Hq - 1)):
+        x = q[b, :, h].double()
+        x = x * c + torch.cat([-x[:, 64:], x[:, :64]], 1) * s
+        sc = x @ k[b, :, h // (Hq // Hkv)].double().t() * D ** -0.5
+        i = torch.arange(L, device=device)
+        sc = sc.masked_fill(torch.arange(N, device=device)[None] > i[:, None] + N - L, float('-inf'))
+        assert_close(to_np(out[b, :, h]), (torch.softmax(sc, -1) @ v[b, :, h // (Hq // Hkv)].double()).cpu().numpy(),
+                     what=f'head {h}')
+
+
 def test_short_and_ragged_calls_run_whole(device):
     """No split where the runs would be short, the items fill the CUs evenly
     enough, or the key counts are known on the device only."""

@@ -30,7 +30,8 @@ def exact_rounded(x):
 
 
 @pytest.mark.parametrize('K,N,B,n', [(32, 16, 1, 1), (160, 48, 2, 33), (1056, 272, 3, 31), (4096, 256, 1, 64),
-                                     (5120, 384, 4, 300), (96, 1040, 1, 700)])
+                                     (5120, 384, 4, 300), (96, 1040, 1, 700), (4096, 64, 1, 4),
+                                     (4096, 64, 5, 1), (1056, 48, 1, 36), (1056, 48, 1, 37)])
 def test_tile_edges(device, K, N, B, n):
     from slimkv_amd import kernels
     x, w, rows = _problem(device, K, N, B, n + 9, n)

@@ -8,6 +8,8 @@ import os
 from functools import lru_cache
 from pathlib import Path
 
+import torch
+
 LIBRARY = Path(__file__).resolve().parent / 'libslimkv_hip.so'
 
 c_i64 = ctypes.c_int64
@@ -365,11 +367,17 @@ def check(code):
         raise SlimKVError(f'slimkv_hip error {code}: {message}')
 
 
+_gpu_index = {}       # torch.device with an index -> that index, for devices seen as GPUs
+
+
 def stream_handle(device):
     """Address of torch's current stream on `device` (what
-    torch.cuda.current_stream takes); a tensor's device is looked up without
+    torch.cuda.current_stream takes); a device seen before is looked up without
     building a Stream object for it."""
-    import torch
-    if isinstance(device, torch.device) and device.type == 'cuda' and device.index is not None:
-        return torch._C._cuda_getCurrentRawStream(device.index)
-    return torch.cuda.current_stream(device).cuda_stream
+    index = _gpu_index.get(device)
+    if index is not None:
+        return torch._C._cuda_getCurrentRawStream(index)
+    stream = torch.cuda.current_stream(device)
+    if isinstance(device, torch.device) and device.index is not None:
+        _gpu_index[device] = device.index
+    return stream.cuda_stream

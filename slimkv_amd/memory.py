@@ -6,6 +6,7 @@ and slimkv/memory.py:999-1007 (cat_tensor); `materialize` builds the full-dim
 place instead of concatenating.
 """
 import torch
+from torch.autograd.forward_ad import unpack_dual
 
 from . import kernels
 
@@ -49,20 +50,20 @@ def _flat_latents(latent):
     return latent.transpose(1, 2).reshape(batch, length, heads * dim)
 
 
-def _differentiated(part):
-    """Whether torch's copy of `part` would record a gradient or carry a
-    forward-mode tangent."""
-    return (part.requires_grad and torch.is_grad_enabled()) or torch.autograd.forward_ad.unpack_dual(part).tangent is not None
-
-
 def _copyable(part, out):
     """Whether a full-width part can be copied as rows: plain memory of out's
-    type, device, batch and heads, 16-byte rows, no derivative to carry."""
-    if type(part) not in (torch.Tensor, torch.nn.Parameter) or part.is_neg() or _differentiated(part):
+    type, device, batch and heads, 16-byte rows, no gradient to record and no
+    forward-mode tangent to carry."""
+    if type(part) is not torch.Tensor and type(part) is not torch.nn.Parameter:
         return False
-    return (part.dtype == out.dtype == torch.bfloat16 and part.device == out.device
-            and part.shape[:2] == out.shape[:2] and part.shape[3] == out.shape[3] and part.stride(3) == 1
-            and part.data_ptr() % 16 == 0 and not any(s % 8 for s in part.stride()[:3]))
+    if part.dtype is not torch.bfloat16 or out.dtype is not torch.bfloat16 or part.dim() != 4 or part.device != out.device:
+        return False
+    (batch, heads, _, dim), (sb, sh, sn, sd) = part.shape, part.stride()
+    if (batch, heads, dim) != (out.shape[0], out.shape[1], out.shape[3]) or sd != 1 or (sb | sh | sn) % 8:
+        return False
+    if part.data_ptr() % 16 or part.is_neg() or (part.requires_grad and torch.is_grad_enabled()):
+        return False
+    return unpack_dual(part).tangent is None
 
 
 class ReconstructionCache:

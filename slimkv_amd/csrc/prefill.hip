@@ -527,6 +527,8 @@ PrefillSplit plan_split(const slimkv_prefill_attention_args* a) {
     PrefillSplit sp{};
     if (a->seqlens_k || a->keys <= 0 || a->batch <= 0 || a->queries <= 0 || (a->causal && a->keys < a->queries)) return sp;
     const int64_t qblocks = (a->queries + kQRows - 1) / kQRows;
+    const int cu = device_cu_count(), slots = 2 * cu / kXcds * kXcds;
+    if (a->batch > 2 * cu || a->heads > 2 * cu || qblocks > 2 * cu || a->batch * a->heads * qblocks > 2 * cu) return sp;
     int64_t tiles = 0, longest = 0;
     for (int64_t qb = 0; qb < qblocks; ++qb) {
         const int64_t k_end = a->causal ? std::min<int64_t>(a->keys, std::min<int64_t>(qb * kQRows + kQRows, a->queries) + a->keys - a->queries)
@@ -534,9 +536,8 @@ PrefillSplit plan_split(const slimkv_prefill_attention_args* a) {
         longest = (k_end + kKeys - 1) / kKeys;
         tiles += longest;
     }
-    const int cu = device_cu_count(), slots = 2 * cu / kXcds * kXcds;
     const int64_t items = a->batch * a->heads * qblocks, total = a->batch * a->heads * tiles;
-    if (slots < kXcds || tiles > (1 << 30) || total < slots || items > 2 * cu) return sp;
+    if (slots < kXcds || tiles > (1 << 30) || total < slots) return sp;
     const double whole = longest * (items <= cu ? 1.55 : 1.9 + 0.4 * (double)(items - cu) / cu);
     const double split = 15 + 0.035 * (double)(slots + items) + 2.3 * (double)total / slots;
     if (split > 0.93 * whole) return sp;

@@ -528,7 +528,12 @@ def reconstruct_with_rows(latent, weight, bias, out, first_row, parts, *, block_
     more).  Returns out."""
     _need_device(*(t for _, t in parts))
     _need_bf16(*(t for _, t in parts))
+    if out.dim() != 4 or latent.dim() != 3 or latent.shape[0] != out.shape[0] or \
+            weight.shape != (out.shape[1] * out.shape[3], latent.shape[2]):
+        raise ValueError('expected latent rows [B, n, R], weight [Hkv*D, R] and out [B, Hkv, total, D]')
     heads, n = out.shape[1], latent.shape[1]
+    if first_row < 0 or first_row + n > out.shape[2]:
+        raise ValueError('the rebuilt rows must lie inside the output')
     a, _, keep = _reconstruct_args(latent, weight, bias, heads, out[:, :, first_row:first_row + n].transpose(1, 2), None,
                                    None, None, None, block_diagonal)
     copies = (_lib.RowCopy * len(parts))()

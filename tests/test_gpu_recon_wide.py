@@ -168,3 +168,18 @@ def test_decode_over_rebuilt_rotated_keys(device, R, B, n, repeats):
     sc = x @ key.transpose(-1, -2).contiguous() * D ** -0.5
     assert_close(to_np(out[:, 0]), (torch.softmax(sc, -1) @ value.contiguous()).reshape(B, Hq, D).cpu().numpy(),
                  what=f'width {R}')
+
+
+def test_rows_outside_the_output_are_refused(device):
+    from slimkv_amd import kernels
+    lat = torch.zeros(1, 20, 256, dtype=torch.bfloat16, device=device)
+    w = torch.zeros(HKV * D, 256, dtype=torch.bfloat16, device=device)
+    out = torch.zeros(1, HKV, 24, D, dtype=torch.bfloat16, device=device)
+    part = torch.ones(1, HKV, 4, D, dtype=torch.bfloat16, device=device)
+    kernels.reconstruct_with_rows(lat, w, None, out, 4, [(0, part)])
+    for first, rows, weight, target in ((5, 0, w, out), (-1, 0, w, out), (4, 21, w, out), (4, -1, w, out),
+                                        (4, 0, w[:, :128], out), (4, 0, w, out[..., :64]),
+                                        (4, 0, w, out.expand(2, -1, -1, -1))):
+        with pytest.raises(ValueError):
+            kernels.reconstruct_with_rows(lat, weight, None, target, first, [(rows, part)])
+    assert bool((out[:, :, :4] == 1).all()) and bool((out[:, :, 4:] == 0).all())

@@ -3257,7 +3257,8 @@ int plan_recon(const slimkv_recon_decode_args* r, ReconPlan* p) {
     if (B <= 0 || Lq <= 0 || Lq > 2 || Hq <= 0 || Hkv <= 0 || Hq % Hkv) return fail(SLIMKV_EINVAL, "invalid sizes");
     if (D != 128) return fail(SLIMKV_EUNSUP, "reconstruction decode is built for head_dim 128");
     if (a->raw_keys <= 0 || a->lat_keys < 0) return fail(SLIMKV_EINVAL, "invalid key counts");
-    if (!ptr_aligned16(a->q) || !aligned8(a->q_sb) || !aligned8(a->q_sl) || !aligned8(a->q_sh))
+    if (!ptr_aligned16(a->q) || (B > 1 && !aligned8(a->q_sb)) || (Lq > 1 && !aligned8(a->q_sl)) ||
+        (Hq > 1 && !aligned8(a->q_sh)))
         return fail(SLIMKV_EINVAL, "query rows must be 16-byte aligned");
     if (a->lat_keys > 0 && (!a->lat_k || !a->lat_v)) return fail(SLIMKV_EINVAL, "null latent pointer");
     if (r->beacon_positions && B > 1 && r->bpos_sb < a->lat_keys)

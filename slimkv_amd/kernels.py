@@ -593,7 +593,7 @@ def recon_decode(q, raw_k, raw_v, lat_k, lat_v, up_k, up_v, scale, *, beacon_pos
     rotated beacon keys are rebuilt in fp32 and rounded once, unless
     reference_rounding asks for the reference's bf16 steps (the bits
     ReconstructionCache.materialize writes, modeling_llama.py:1405-1483)."""
-    if any(s % 8 for s in q.stride()[:3]):
+    if any(n > 1 and s % 8 for n, s in zip(q.shape[:3], q.stride())):
         q = q.contiguous()
     base, out, lse, keep = _latent_args(q, raw_k, raw_v, lat_k, lat_v, up_k, up_v, scale, up_k_bias, up_v_bias,
                                         block_diagonal, lat_causal, q_positions, cos, sin, raw_lengths,

@@ -99,3 +99,7 @@ def test_rows_off_a_16_byte_boundary_are_refused():
         for name, value in change.items():
             setattr(r.base, name, value)
         assert lib.slimkv_recon_decode_workspace(ctypes.byref(r)) == 0
+    r = _lib.ReconDecodeArgs()                  # strides of dimensions of one element do not count
+    r.base = latent_args(1, 32, 700, 256, 256)
+    r.base.q_sb = r.base.q_sl = 3
+    assert lib.slimkv_recon_decode_workspace(ctypes.byref(r)) > 0
